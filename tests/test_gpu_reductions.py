@@ -1,0 +1,79 @@
+"""Slicing and moment reductions at the sizes where their loops change: one
+macroparticle, a workgroup's edge, a full grid's edge, more than one unrolled
+step, arrays that are not 16-byte aligned, and masks of lost particles."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+# pairs of a workgroup, of a full grid (256 x 1024) and of one unrolled step
+# of it (4 pairs a thread), and their neighbours
+SIZES = [1, 2, 3, 1023, 2047, 2049, 2 * 262144 + 1, 8 * 262144 - 1, 8 * 262144 + 3]
+
+
+def _bunch(n, seed):
+    rng = np.random.default_rng(seed)
+    return rng.normal(1.25e-9, 0.25e-9, n), rng.normal(3e5, 1e8, n)
+
+
+def _device(a, shift):
+    """A copy on the GPU that starts `shift` elements after an aligned address."""
+    import torch
+
+    buf = torch.zeros(len(a) + shift, dtype=torch.from_numpy(a).dtype, device="cuda")
+    buf[shift:] = torch.from_numpy(a).cuda()
+    return buf[shift:]
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("shift", [0, 1])
+def test_histograms_at_loop_edges(n, shift):
+    import torch
+
+    from blond_amd.utils import bmath as bm
+
+    dt, _ = _bunch(n, n)
+    lib = orc.oracle_lib()
+    for n_slices in (1, 777):
+        ref = np.zeros(n_slices)
+        lib.slice_beam(dt, ref, 0.0, 2.5e-9)
+        got = torch.full((n_slices,), 7.0, dtype=torch.float64, device="cuda")
+        bm.slice_beam(_device(dt, shift), got, 0.0, 2.5e-9)
+        assert np.array_equal(got.cpu().numpy(), ref)
+    ref = np.zeros(777)
+    lib.slice_smooth(dt, ref, 0.0, 2.5e-9)
+    got = torch.full((777,), 7.0, dtype=torch.float64, device="cuda")
+    bm.slice_smooth(_device(dt, shift), got, 0.0, 2.5e-9)
+    # each weight is rounded to 2^-S with S >= 61 - ceil(log2 n) - 1 or 44,
+    # and a bin sums at most n of them; the oracle's running sum rounds n times
+    tol = n * 2.0 ** -(min(44, 60 - int(np.ceil(np.log2(max(n, 2)))))) + n * 2.0 ** -52 * ref.max()
+    assert np.max(np.abs(got.cpu().numpy() - ref)) <= max(tol, 1e-300)
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("lost", [None, "some", "all"])
+def test_moments_at_loop_edges(n, shift, lost):
+    from blond_amd.utils import bmath as bm
+
+    dt, dE = _bunch(n, n)
+    ids = np.arange(1, n + 1)
+    if lost == "some":
+        ids[::3] = 0
+    elif lost == "all":
+        ids[:] = 0
+    alive = ids != 0
+    got = bm.beam_statistics(_device(dt, shift), _device(dE, shift),
+                             None if lost is None else _device(ids, shift))
+    assert got[0] == alive.sum()
+    if not alive.any():
+        assert got[1:] == (0.0, 0.0, 0.0, 0.0)
+        return
+    # sums of k terms of size |x|: a few roundings of the largest partial sum
+    x, e = dt[alive], dE[alive]
+    eps = 64 * 2.0 ** -52
+    for mean, sigma, v in ((got[1], got[2], x), (got[3], got[4], e)):
+        assert abs(mean - np.mean(v)) <= eps * np.mean(np.abs(v))
+        assert abs(sigma - np.std(v)) <= eps * max(np.std(v), np.mean(np.abs(v)))
