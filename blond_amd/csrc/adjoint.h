@@ -14,11 +14,13 @@ namespace blmi {
 // Largest slice count of the differentiable tracker (each workgroup of its
 // induced-voltage kernels holds the profile, the wake and the adjoints).
 constexpr int kAdjMaxSlices = 1024;
-constexpr int kAdjCopies = 16;  // copies of the global deposit / adjoint accumulators
+constexpr int kAdjCopies = 8;  // copies of the global deposit / adjoint accumulators
+constexpr int kAdjRing = 3;    // accumulators in rotation (read, added to, cleared)
 
 struct Adjoint {
     int device = 0;
     int64_t n = 0;
+    int64_t np = 0;            // n rounded up to even: the stride of a state's arrays
     int n_rf = 0, n_turns = 0, n_slices = 0, every = 50;
     int64_t n_fft = 0;
     double charge = 1.0, scale = 0.0;
@@ -32,20 +34,22 @@ struct Adjoint {
     double *d_rf = nullptr, *d_acc = nullptr;
     DriftCoeffs<double> *d_drift = nullptr;
     // coordinates: initial (owned copy), working, checkpoints, recompute slots
-    double *d_x0 = nullptr;    // [2][n]: dt, dE at turn 0
-    double *d_work = nullptr;  // [2][n]
-    double *d_ckpt = nullptr;  // [n_ckpt][2][n]
-    double *d_slots = nullptr; // [every][2][n]
-    double *d_lam = nullptr;   // [2][n]: adjoints of dt, dE
+    double *d_x0 = nullptr;    // [2][np]: dt, dE at turn 0
+    double *d_work = nullptr;  // [2][np]
+    double *d_ckpt = nullptr;  // [n_ckpt][2][np] (entry 0 unused: d_x0 holds turn 0)
+    double *d_slots = nullptr; // [every][2][np]
+    double *d_lam = nullptr;   // [2][np]: adjoints of dt, dE
     // slice axis
-    unsigned long long *d_dep = nullptr;  // [2 parity][copies][n_slices] fixed-point deposit
+    unsigned long long *d_dep = nullptr;  // [kAdjRing][copies][n_slices] fixed-point deposit
     double *d_prof = nullptr;  // [n_turns + 1][n_slices] profiles p_t
     double *d_vt = nullptr;    // [n_turns + 1][n_slices] induced voltage V_t
     double *d_g = nullptr;     // wake g = irfft(Z) [n_fft]
-    double *d_lv = nullptr;    // [2 parity][copies][n_slices] adjoint of V_t (accumulated)
+    double *d_lv = nullptr;    // [kAdjRing][copies][n_slices] adjoint of V_t (accumulated)
+    double *d_lvh = nullptr;   // [n_turns][n_slices] adjoint of V_t, every turn
     double *d_lp = nullptr;    // [n_slices] adjoint of the profile
     double *d_corr = nullptr;  // [n_fft] sum_t sum_i lambda_V,t[i] p_t[(i - m) mod n_fft]
-    double *d_gpart = nullptr; // [n_turns][grid][2 n_rf] per-workgroup RF gradient sums
+    double *d_corr_part = nullptr;  // rows of d_corr before their sum
+    double *d_gpart = nullptr; // [grid][2 n_rf] per-workgroup RF gradient sums
     int grid = 0, block = 256;
     bool forward_done = false;
     int forward_turns = 0;
