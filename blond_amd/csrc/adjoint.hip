@@ -804,8 +804,7 @@ __global__ void __launch_bounds__(kAdjBlock) adj_reverse_kernel(const double *__
 #pragma unroll
     for (int j = 0; j < 2 * kAdjMaxRf; ++j) {
         if (j < 2 * a.n_rf) {
-            double v = gsum[j];
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+            const double v = wave_sum(gsum[j]);
             if (lane == 0) red[wid][j] = v;
         }
     }

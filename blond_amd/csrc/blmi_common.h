@@ -284,9 +284,12 @@ template <> struct TrigTab<float> {
 // float): the voltage and the bin centres are float arrays there, so V is
 // rounded to float and the scale and each entry are formed in float, in the
 // same order, and stored exactly as doubles.
+__device__ __forceinline__ double interp_inv_bw(double bc_first, double bc_last, int ns, bool f32) {
+    if (f32) return (double)((float)(ns - 1) / ((float)bc_last - (float)bc_first));
+    return (double)(ns - 1) / (bc_last - bc_first);
+}
 __device__ __forceinline__ double interp_inv_bw(const double *bc, int ns, bool f32) {
-    if (f32) return (double)((float)(ns - 1) / ((float)bc[ns - 1] - (float)bc[0]));
-    return (double)(ns - 1) / (bc[ns - 1] - bc[0]);
+    return interp_inv_bw(bc[0], bc[ns - 1], ns, f32);
 }
 
 __device__ __forceinline__ double2 interp_entry(double v0, double v1, double bcb, double charge,
@@ -309,6 +312,49 @@ __device__ __forceinline__ void store_interp_entry(double2 *tab, int i, double2 
         reinterpret_cast<float2 *>(tab)[i] = make_float2((float)e.x, (float)e.y);
     else
         tab[i] = e;
+}
+
+// ---------------------------------------------------------------------------
+// Lane exchanges in registers (DPP and gfx950's lane swaps): a butterfly step
+// of a double is two or three vector instructions, where __shfl_xor sends both
+// words through the LDS crossbar and waits for them.
+// ---------------------------------------------------------------------------
+// The value of lane ^ BIT, BIT in {1, 2, 4, 8}.
+template <int BIT>
+__device__ __forceinline__ int lane_xor32(int v) {
+    static_assert(BIT == 1 || BIT == 2 || BIT == 4 || BIT == 8, "within a row of 16 lanes");
+    if constexpr (BIT == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);
+    if constexpr (BIT == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);
+    if constexpr (BIT == 8) return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true);
+    // lane ^ 7 (half-row mirror), then ^ 3 (reversed quads)
+    const int m = __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);
+    return __builtin_amdgcn_update_dpp(0, m, 0x1B, 0xf, 0xf, true);
+}
+template <int BIT>
+__device__ __forceinline__ double lane_xor(double v) {
+    return __hiloint2double(lane_xor32<BIT>(__double2hiint(v)), lane_xor32<BIT>(__double2loint(v)));
+}
+// A halving step over lane bit 5 (4): lanes with the bit clear get a's sum
+// over the pair of lanes, the others b's.  With a == b every lane gets it.
+__device__ __forceinline__ double halve32(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ double halve16(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+// Sum over the wavefront in every lane (the xor butterfly from bit 5 down).
+__device__ __forceinline__ double wave_sum(double v) {
+    v = halve32(v, v);
+    v = halve16(v, v);
+    v += lane_xor<8>(v);
+    v += lane_xor<4>(v);
+    v += lane_xor<2>(v);
+    v += lane_xor<1>(v);
+    return v;
 }
 
 // Agent-scope atomics (all XCDs of the device see one coherent value).

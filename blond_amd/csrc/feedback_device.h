@@ -13,10 +13,8 @@ constexpr int kFbBlock = 1024;
 // valid in thread 0.
 __device__ inline void block_sum2(double &a, double &b) {
     __shared__ double wa[kFbBlock / kWave], wb[kFbBlock / kWave];
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        a += __shfl_xor(a, off);
-        b += __shfl_xor(b, off);
-    }
+    a = wave_sum(a);
+    b = wave_sum(b);
     const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
     if (lane == 0) {
         wa[w] = a;

@@ -508,6 +508,14 @@ __global__ void __launch_bounds__(FL > 0 ? kLdsWaveThreads : 1024)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int conv_pad(int k) { return k + (k >> 3); }
 
+// Values of the epilogue that a workgroup reads from memory at its start, so
+// that no round trip follows the products.
+struct DirectTail {
+    double bc_first = 0.0, bc_last = 0.0;  // bin centres 0 and n_slices - 1
+    double bc_i = 0.0;                     // bin centre of this thread's output
+    double h = 0.0, coef = 0.0;            // inductive term: bc[1] - bc[0], coefficient
+};
+
 // The wake step of the turn on this workgroup's outputs, as the engine's
 // separate wake step computes it (wake.hip): the memory after the turn
 // mem(i) = interp(old memory one revolution later) + V(i) for i < n_add
@@ -519,7 +527,7 @@ template <int C>
 __device__ __forceinline__ void direct_wake_epilogue(const InducedArgs &a, const double *q,
                                                      const double *vout, double *memv,
                                                      double mprev, int t, int i0,
-                                                     unsigned *cclr) {
+                                                     unsigned *cclr, const DirectTail &tail) {
     const WakeArgs &w = a.wk;
     const int ns = a.n_slices;
     if ((int)threadIdx.x <= C) {
@@ -535,15 +543,13 @@ __device__ __forceinline__ void direct_wake_epilogue(const InducedArgs &a, const
     if ((int)threadIdx.x >= C) return;
     const int i = i0 + threadIdx.x;
     if (i >= ns) return;
-    const double coef = w.ind_coef ? w.ind_coef[t] : 0.0;
     auto prof = [&](int k) -> double { return q[conv_pad(ns - 1 - k)]; };
     auto total = [&](int c, int j) -> double {
         double v = 0.0;
         v = v + memv[c];
         if (w.ind_coef) {
-            const double d = profile_derivative_at(prof, w.bc, ns, w.bc[1] - w.bc[0],
-                                                   w.deriv_mode, j);
-            v = v + (-(coef * d));
+            const double d = profile_derivative_at(prof, w.bc, ns, tail.h, w.deriv_mode, j);
+            v = v + (-(tail.coef * d));
         }
         return v;
     };
@@ -553,22 +559,21 @@ __device__ __forceinline__ void direct_wake_epilogue(const InducedArgs &a, const
     if (cclr)
         for (int g = 0; g < a.groups; ++g) cclr[(size_t)g * ns + i] = 0u;
     if (a.tab) {
-        const double inv_bw = (double)(ns - 1) / (a.bc[ns - 1] - a.bc[0]);
+        const double inv_bw = interp_inv_bw(tail.bc_first, tail.bc_last, ns, false);
         if (i == 0) {
-            a.tab_params[0] = a.bc[0];
+            a.tab_params[0] = tail.bc_first;
             a.tab_params[1] = inv_bw;
         }
         if (i < ns - 1) {
             const double vn = total(threadIdx.x + 1, i + 1);
-            const double k = a.charge * (vn - vi) * inv_bw;
-            a.tab[i] = make_double2(k, (a.charge * vi - a.bc[i] * k) + 0.0);
+            a.tab[i] = interp_entry(vi, vn, tail.bc_i, a.charge, inv_bw, false);
         }
     }
 }
 
 template <int C, int TH, int CHUNK>
 __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
-    static_assert(C >= 2 && C <= 32 && (C & (C - 1)) == 0, "C is a power of two up to 32");
+    static_assert(C >= 4 && C <= 32 && (C & (C - 1)) == 0, "C is a power of two, 4 to 32");
     static_assert(CHUNK % 8 == 0, "a thread's samples start on a pad period");
     const int nfb = a.with_fb ? a.fb.n_parts : 0;
     if ((int)blockIdx.x < nfb) {
@@ -585,6 +590,13 @@ __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
     // with the loop, workgroups 0 .. nfb - 1 run it (dispatched first: they
     // are the longest) and workgroup b >= nfb takes outputs of b - nfb
     const int i0 = (blockIdx.x - nfb) * C;
+    DirectTail tl;
+    if (a.tab) {
+        tl.bc_first = a.bc[0];
+        tl.bc_last = a.bc[ns - 1];
+        const int i = i0 + (int)threadIdx.x;
+        if ((int)threadIdx.x < C && i < ns) tl.bc_i = a.bc[i];
+    }
     // wake step: the previous memory's value one revolution later at this
     // workgroup's outputs (impedance.py:536-550), read first so that its
     // dependent loads overlap the staging and the products below
@@ -596,23 +608,31 @@ __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
         if ((int)threadIdx.x <= C && i < a.wk.n_mem)
             mprev = mtw_value((wt & 1) ? a.wk.mem1 : a.wk.mem0, a.wk.time, a.wk.n_mem,
                               a.wk.t_rev[wt], i);
+        if (a.wk.ind_coef) {
+            tl.h = a.wk.bc[1] - a.wk.bc[0];
+            tl.coef = a.wk.ind_coef[wt];
+        }
     }
     const int lim = a.n_out + ns - 1;  // gl entries used (host checks gl_len)
     const int nq = (ns + kSpan - 1) / kSpan * kSpan;
     double *q = conv_lds;                  // q[pad(m)], zero for m >= ns
     double *wv = conv_lds + conv_pad(nq);  // wv[pad(k)] = gl[i0 + k], k < nq + C
+    // up to a span of 2048 samples both parities' counts are read and the
+    // turn's chosen when they arrive, so the turn's load is not waited for first
+    constexpr bool kBoth = kSpan <= 2048;
     const unsigned *cin = nullptr;
     unsigned *cclr = nullptr;
+    bool odd = false;
     if (a.counts0) {
-        const int t = *a.turn_base + a.turn_off;
-        cin = (t & 1) ? a.counts1 : a.counts0;
-        cclr = (t & 1) ? a.counts0 : a.counts1;
+        odd = (*a.turn_base + a.turn_off) & 1;
+        cin = kBoth || !odd ? a.counts0 : a.counts1;
+        cclr = odd ? a.counts0 : a.counts1;
     }
     // Staging in batches of 8 entries per thread: every load of a batch
     // (window, profile, and the window's last C entries with the last batch)
     // is issued before the first LDS store, with clamped in-bounds indexes
     // and the out-of-range values replaced afterwards, so the batch costs
-    // one memory round trip (plus one per extra count copy).
+    // one memory round trip (four copies of the counts at a time).
     constexpr int kStage = 8;
     for (int b = 0; b < nq; b += kStage * TH) {
         double wx[kStage], qx[kStage];
@@ -629,17 +649,33 @@ __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
         const double xt = a.gl[okt ? i0 + kt : 0];
         if (cin) {
             unsigned cs[kStage];
+            // NG copies of the counts at once, all their loads in flight
+            auto copies = [&](auto ng, int g0) {
+                constexpr int NG = decltype(ng)::value;
+                unsigned x[NG][kStage], y[NG][kStage];
+#pragma unroll
+                for (int g = 0; g < NG; ++g)
+#pragma unroll
+                    for (int u = 0; u < kStage; ++u) {
+                        const int m = b + u * TH + (int)threadIdx.x;
+                        const size_t at = (size_t)(g0 + g) * ns + (m < ns ? ns - 1 - m : 0);
+                        x[g][u] = cin[at];
+                        if (kBoth) y[g][u] = a.counts1[at];
+                    }
+#pragma unroll
+                for (int g = 0; g < NG; ++g)
+#pragma unroll
+                    for (int u = 0; u < kStage; ++u) {
+                        const int m = b + u * TH + (int)threadIdx.x;
+                        const unsigned v = kBoth && odd ? y[g][u] : x[g][u];
+                        cs[u] += m < ns ? v : 0u;
+                    }
+            };
 #pragma unroll
             for (int u = 0; u < kStage; ++u) cs[u] = 0u;
-            for (int g = 0; g < a.groups; ++g) {
-                const unsigned *row = cin + (size_t)g * ns;
-#pragma unroll
-                for (int u = 0; u < kStage; ++u) {
-                    const int m = b + u * TH + (int)threadIdx.x;
-                    const unsigned x = row[m < ns ? ns - 1 - m : 0];
-                    cs[u] += m < ns ? x : 0u;
-                }
-            }
+            int g = 0;
+            for (; g + 4 <= a.groups; g += 4) copies(std::integral_constant<int, 4>{}, g);
+            for (; g < a.groups; ++g) copies(std::integral_constant<int, 1>{}, g);
 #pragma unroll
             for (int u = 0; u < kStage; ++u) qx[u] = (double)cs[u];
         } else {
@@ -681,22 +717,32 @@ __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
     // of its sums and adds its partner's copy of them; after log2(C)
     // exchanges a lane holds one sum (index idx) over 64/C lanes' worth
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    int idx = 0, bit = 32;
+    int idx = 0;
 #pragma unroll
-    for (int half = C / 2; half >= 1; half >>= 1) {
-        const bool hi = lane & bit;
+    for (int k = 0; k < C / 2; ++k) acc[k] = halve32(acc[k], acc[k + C / 2]);
 #pragma unroll
-        for (int k = 0; k < half; ++k) {
-            const double send = hi ? acc[k] : acc[k + half];
-            const double keep = hi ? acc[k + half] : acc[k];
-            acc[k] = keep + __shfl_xor(send, bit);
+    for (int k = 0; k < C / 4; ++k) acc[k] = halve16(acc[k], acc[k + C / 4]);
+    idx += (lane & 32 ? C / 2 : 0) + (lane & 16 ? C / 4 : 0);
+    auto exchange = [&](auto bit, auto half) {
+        constexpr int B = decltype(bit)::value, H = decltype(half)::value;
+        const bool hi = lane & B;
+        if constexpr (H >= 1) {
+#pragma unroll
+            for (int k = 0; k < H; ++k) {
+                const double send = hi ? acc[k] : acc[k + H];
+                const double keep = hi ? acc[k + H] : acc[k];
+                acc[k] = keep + lane_xor<B>(send);
+            }
+            if (hi) idx += H;
+        } else {
+            acc[0] += lane_xor<B>(acc[0]);
         }
-        if (hi) idx += half;
-        bit >>= 1;
-    }
-    for (int b = bit; b > 0; b >>= 1) acc[0] += __shfl_xor(acc[0], b);
-    double last = acc[C];
-    for (int off = 32; off > 0; off >>= 1) last += __shfl_xor(last, off);
+    };
+    exchange(std::integral_constant<int, 8>{}, std::integral_constant<int, C / 8>{});
+    exchange(std::integral_constant<int, 4>{}, std::integral_constant<int, C / 16>{});
+    exchange(std::integral_constant<int, 2>{}, std::integral_constant<int, C / 32>{});
+    exchange(std::integral_constant<int, 1>{}, std::integral_constant<int, C / 64>{});
+    const double last = wave_sum(acc[C]);
     if ((lane & (64 / C - 1)) == 0) red[wid][idx] = acc[0];
     if (lane == 0) red[wid][C] = last;
     __syncthreads();
@@ -707,7 +753,7 @@ __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
     }
     __syncthreads();
     if (a.with_wake) {
-        direct_wake_epilogue<C>(a, q, vout, memv, mprev, wt, i0, cclr);
+        direct_wake_epilogue<C>(a, q, vout, memv, mprev, wt, i0, cclr, tl);
         return;
     }
     if (threadIdx.x < C) {
@@ -721,16 +767,16 @@ __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
     }
     if (a.tab) {
         // linear_interp_kick.cpp:33-48 on V (acc = 0 for the induced kick)
-        const double inv_bw = interp_inv_bw(a.bc, ns, a.f32);
+        const double inv_bw = interp_inv_bw(tl.bc_first, tl.bc_last, ns, a.f32);
         if (i0 == 0 && threadIdx.x == 0) {
-            a.tab_params[0] = a.bc[0];
+            a.tab_params[0] = tl.bc_first;
             a.tab_params[1] = inv_bw;
         }
         if (threadIdx.x < C) {
             const int i = i0 + threadIdx.x;
             if (i < ns - 1)
                 store_interp_entry(a.tab, i,
-                                   interp_entry(vout[threadIdx.x], vout[threadIdx.x + 1], a.bc[i],
+                                   interp_entry(vout[threadIdx.x], vout[threadIdx.x + 1], tl.bc_i,
                                                 a.charge, inv_bw, a.f32),
                                    a.f32);
         }
@@ -778,19 +824,28 @@ static int launch_direct_shape(const InducedArgs &a0, hipStream_t s, const Kerne
 }
 
 // Shape of the direct convolution (outputs per workgroup, workgroup size,
-// samples per thread), measured on one MI355X with a 4096-slice profile and
-// its neighbours: 1024 slices 5.0 us (16, 256, 8); 2048 slices 6.1 us and
-// 4096 slices 6.8 us (16, 512, 8); 8192 slices 11.6 us (32, 512, 16).  A
-// multi-turn memory (n_out = 4 x 4096 values of 4096 slices) takes (32, 512,
-// 8): 21.8 against 22.5 us for (16, 512, 8) with its wake step.
+// samples per thread), the launch's time in a turn (HIP events; 200, 500, 1000
+// slices with four count copies):
+//   up to 1024 slices (8, 128, 8) 4.5, 4.4, 4.5 us; (16, 256, 8) 5.1, 5.3, 5.2
+//     (fewer sums to exchange, more CUs); with the beam phase loop, whose sums
+//     take the same workgroup size, (16, 256, 8): 7.5 against 9.0 us
+//   2000 slices (16, 512, 8) 4.9 us, (16, 256, 8) 5.1
+//   4096 slices (16, 512, 8) 5.5 us, (16, 256, 8) 6.4, (8, 512, 8) 8.2
+//   8192 slices (32, 512, 16)
+//   a multi-turn memory, 16384 outputs of 4096 slices with the wake step:
+//     (32, 256, 16) 10.3 us, (32, 512, 8) 13.3, (16, 512, 8) 19.6: the
+//     exchange of a workgroup's sums is paid for once per 32 outputs and
+//     wavefront, so fewer wavefronts with more samples each
 int launch_induced_direct(const InducedArgs &a, hipStream_t s, const KernelEvents &ev) {
     if (!a.gl || a.n_slices < 1 || a.n_out < a.n_slices ||
         (int64_t)a.n_out + a.n_slices - 1 > a.gl_len ||
         (a.tab && a.n_out != a.n_slices && !a.with_wake) ||
         (a.with_wake && (a.wk.n_mem > a.n_out || (a.wk.ind_coef && a.n_slices < 2))))
         return blmi_set_error(BLMI_ERR_ARG, "direct induced voltage: bad arguments");
-    if (a.n_out > a.n_slices && a.n_slices > 1024) return launch_direct_shape<32, 512, 8>(a, s, ev);
-    if (a.n_slices <= 1024) return launch_direct_shape<16, 256, 8>(a, s, ev);
+    if (a.n_out > a.n_slices && a.n_slices > 1024) return launch_direct_shape<32, 256, 16>(a, s, ev);
+    if (a.n_slices <= 1024)
+        return a.with_fb ? launch_direct_shape<16, 256, 8>(a, s, ev)
+                         : launch_direct_shape<8, 128, 8>(a, s, ev);
     if (a.n_slices <= 4096) return launch_direct_shape<16, 512, 8>(a, s, ev);
     return launch_direct_shape<32, 512, 16>(a, s, ev);
 }
