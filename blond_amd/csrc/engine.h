@@ -18,6 +18,8 @@ namespace blmi {
 constexpr int kLdsHistBytes = 131072;    // histogram words in LDS at most
 constexpr int kLdsHistU32Bytes = 65536;  // u32 counts up to this, u16 pairs above
 constexpr int kMaxParticlesPerGroup16 = 65535;
+// slice counts up to which a small bunch takes smaller workgroups
+constexpr int kSmallBlockSlices = 1024;
 // turns a plain-tracking launch takes at most, by default (odd)
 constexpr int kTurnBlockDefault = 25;
 // the particle kernels' sink: 2 pairs (dt, dE) of doubles for each lane of a wavefront
@@ -148,6 +150,7 @@ struct Engine {
     // launch shape (tunable)
     int block_size = 1024;
     int blocks_per_cu = 1;
+    int launch_block() const;      // the workgroup size launched: block_size or less
     // plain tracking: at most this many turns per particle-kernel launch
     // (the particles stay in registers between them; 1 = a launch a turn)
     int turn_block = kTurnBlockDefault;

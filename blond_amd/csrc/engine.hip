@@ -100,19 +100,25 @@ struct TurnArgs {
 };
 
 // Workgroup sums of the four moment accumulators in a fixed order (wavefront
-// butterfly, then wavefronts in index order), written by thread 0.
+// butterfly, then wavefronts in index order), written by thread 0.  The first
+// two exchanges halve the sums a lane carries (it keeps two of the four, then
+// one, and adds its partner's), so the butterfly is 7 exchanges and not 24:
+// the same pairs are added, and the sums are the same bits.
 __device__ __forceinline__ void stats_flush(double s[4], double *__restrict__ out) {
     __shared__ double wred[1024 / kWave][4];
-    for (int k = 0; k < 4; ++k)
-        for (int off = kWave / 2; off > 0; off >>= 1) s[k] += __shfl_xor(s[k], off);
     const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
-    if (lane == 0)
-        for (int k = 0; k < 4; ++k) wred[w][k] = s[k];
+    double v = halve16(halve32(s[0], s[2]), halve32(s[1], s[3]));
+    v += lane_xor<8>(v);
+    v += lane_xor<4>(v);
+    v += lane_xor<2>(v);
+    v += lane_xor<1>(v);
+    // lanes 0, 16, 32, 48 hold sums 0, 1, 2, 3
+    if ((lane & 15) == 0) wred[w][lane >> 4] = v;
     __syncthreads();
     if (threadIdx.x < 4) {
-        double v = 0.0;
-        for (int q = 0; q < (int)blockDim.x / kWave; ++q) v += wred[q][threadIdx.x];
-        out[threadIdx.x] = v;
+        double t = 0.0;
+        for (int q = 0; q < (int)blockDim.x / kWave; ++q) t += wred[q][threadIdx.x];
+        out[threadIdx.x] = t;
     }
 }
 
@@ -389,11 +395,11 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
     with_rf_count(a.n_rf, [&](auto nrf) {
     rfp.template pin<decltype(nrf)::value>();
     pin_constants();
-    // one pair: RF kick, interpolated kick, drift, store, count; then the
-    // other slot's table loads and this slot's reload two pairs ahead
+    // one pair: RF kick, interpolated kick, drift, store, count; and (more)
+    // the other slot's table loads and this slot's reload two pairs ahead
     V2 *const sink = reinterpret_cast<V2 *>(a.sink) + 2 * (threadIdx.x % kWave);
-    auto pair = [&](V2 &x, V2 &e, Tab &g0, Tab &g1, const V2 &xo, Tab &go0, Tab &go1,
-                    int64_t i) {
+    auto pair = [&](auto more, V2 &x, V2 &e, Tab &g0, Tab &g1, const V2 &xo, Tab &go0,
+                    Tab &go1, int64_t i) {
         const bool own = i < n2;
         int b0 = finish(x.x, e.x, g0, nrf);
         int b1 = finish(x.y, e.y, g1, nrf);
@@ -419,19 +425,21 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         } else {
             b0 = b1 = -1;
         }
-        go0 = gather(xo.x);
-        go1 = gather(xo.y);
-        const int64_t j = clamp(i + 2 * stride);
-        if constexpr (NT) {
-            const NV2 xv =
-                __builtin_nontemporal_load(reinterpret_cast<GlobalPtr<const NV2>>((uint64_t)dt) + j);
-            const NV2 ev =
-                __builtin_nontemporal_load(reinterpret_cast<GlobalPtr<const NV2>>((uint64_t)dE) + j);
-            x = V2{xv.x, xv.y};
-            e = V2{ev.x, ev.y};
-        } else {
-            x = reinterpret_cast<const V2 *>(dt)[j];
-            e = reinterpret_cast<const V2 *>(dE)[j];
+        if constexpr (decltype(more)::value) {
+            go0 = gather(xo.x);
+            go1 = gather(xo.y);
+            const int64_t j = clamp(i + 2 * stride);
+            if constexpr (NT) {
+                const NV2 xv =
+                    __builtin_nontemporal_load(reinterpret_cast<GlobalPtr<const NV2>>((uint64_t)dt) + j);
+                const NV2 ev =
+                    __builtin_nontemporal_load(reinterpret_cast<GlobalPtr<const NV2>>((uint64_t)dE) + j);
+                x = V2{xv.x, xv.y};
+                e = V2{ev.x, ev.y};
+            } else {
+                x = reinterpret_cast<const V2 *>(dt)[j];
+                e = reinterpret_cast<const V2 *>(dE)[j];
+            }
         }
         count(b0);
         count(b1);
@@ -441,12 +449,15 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         xb = reinterpret_cast<const V2 *>(dt)[clamp(i_first + stride)];
         eb = reinterpret_cast<const V2 *>(dE)[clamp(i_first + stride)];
         // both slots every iteration, no exit between them (a branch there
-        // would again leave the waits conservative): with an odd count the
-        // last iteration's second pair is past every lane's end and sunk
-        for (int64_t k = 0; k < iters; k += 2) {
-            pair(xa, ea, ga0, ga1, xb, gb0, gb1, i_first + k * stride);
-            pair(xb, eb, gb0, gb1, xa, ga0, ga1, i_first + (k + 1) * stride);
+        // would again leave the waits conservative); an odd count's last pair
+        // after the loop
+        constexpr std::true_type more{};
+        for (int64_t k = 0; k + 1 < iters; k += 2) {
+            pair(more, xa, ea, ga0, ga1, xb, gb0, gb1, i_first + k * stride);
+            pair(more, xb, eb, gb0, gb1, xa, ga0, ga1, i_first + (k + 1) * stride);
         }
+        if (iters & 1)
+            pair(std::false_type{}, xa, ea, ga0, ga1, xb, gb0, gb1, i_first + (iters - 1) * stride);
     }
     if ((n & 1) && blockIdx.x == gridDim.x - 1 && threadIdx.x < 64) {
         // odd tail: the first wavefront of the last block takes part in the
@@ -1076,6 +1087,19 @@ int Engine::get_turn(int *turn) {
     return BLMI_OK;
 }
 
+// The particle kernels' workgroup: the configured size, halved down to 256
+// threads while a thread still takes at most two pairs, so that a small bunch
+// spreads over all CUs (moderate slice counts: with few threads the table's
+// staging and the histogram's clearing would dominate).  Turn kernel with 500
+// slices, 1024 threads against this: 5e4 macroparticles 6.4 / 5.1 us, 2e5 7.0 /
+// 6.4 us, 5e5 8.9 / 7.5 us.
+int Engine::launch_block() const {
+    const int64_t wgs = (int64_t)device_cu_count() * blocks_per_cu, pairs = (n + 1) / 2;
+    int b = block_size;
+    while (n_slices <= kSmallBlockSlices && b >= 512 && pairs <= wgs * b) b /= 2;
+    return b;
+}
+
 int Engine::hist_layout(int block, int *grid_out, size_t *lds_out) const {
     int grid = device_cu_count() * blocks_per_cu;
     const int64_t n2 = n / 2;
@@ -1126,7 +1150,7 @@ int Engine::ensure_partials() {
     if (n_slices <= 0 || !d_counts || ordered()) return BLMI_OK;
     int grid = 0;
     size_t lds = 0;
-    if (hist_layout(block_size, &grid, &lds) != 2) return BLMI_OK;
+    if (hist_layout(launch_block(), &grid, &lds) != 2) return BLMI_OK;
     const size_t need = sizeof(unsigned) * (size_t)grid * hist_words(2, n_slices);
     if (need > partials_bytes) {
         invalidate_graph();  // a captured graph holds the old rows
@@ -1147,7 +1171,7 @@ bool Engine::part_perm(int *shift, int *lshift, int *m1_lo) const {
         return false;
     int grid = 0;
     size_t lds = 0;
-    if (hist_layout(block_size, &grid, &lds) != 2) return false;
+    if (hist_layout(launch_block(), &grid, &lds) != 2) return false;
     const int W = hist_words(2, n_slices);
     const int M2 = plan2.M2;
     if (M2 < 2 || (M2 & (M2 - 1)) || W % M2) return false;
@@ -1185,7 +1209,7 @@ int Engine::launch_reduce(hipStream_t s, int off) {
     if (part_perm(&ps, &pl)) return BLMI_OK;  // the four-step's first pass sums the rows
     int grid = 0;
     size_t lds = 0;
-    if (hist_layout(block_size, &grid, &lds) != 2) return BLMI_OK;
+    if (hist_layout(launch_block(), &grid, &lds) != 2) return BLMI_OK;
     const int W = hist_words(2, n_slices);
     hipLaunchKernelGGL(partials_reduce_kernel, dim3((W + kRedWords - 1) / kRedWords), dim3(512), 0,
                        s, d_partials, grid, W, d_base, off, d_counts,
@@ -1212,7 +1236,7 @@ static int launch_prime(Engine *e, const T *x, T cl, T ibw, int mode, int grid, 
                                  : (const void *)prime_hist_kernel<T, 0>;
     int rc = lds_attribute(fn, lds);
     if (rc) return rc;
-    const int blk = e->block_size;
+    const int blk = e->launch_block();
     if (mode == 2)
         hipLaunchKernelGGL((prime_hist_kernel<T, 2>), dim3(grid), dim3(blk), lds, s, x, e->n,
                            e->d_base, e->d_counts, c1, e->n_slices, cl, ibw, e->d_partials, W,
@@ -1304,7 +1328,7 @@ int Engine::prime(hipStream_t s) {
     if (rc) return rc;
     int grid = 0;
     size_t lds = 0;
-    int mode = hist_layout(block_size, &grid, &lds);
+    int mode = hist_layout(launch_block(), &grid, &lds);
     if (mode == 2 && ordered()) {
         // no partial rows in the ordered mode: count with device atomics
         mode = 0;
@@ -1407,7 +1431,7 @@ static int launch_turn_t(const Engine &e, T *x, T *de, const T *rf, const T *acc
     a.sink = e.d_sink;
     int grid = 0;
     size_t lds = 0;
-    int ldsh = e.hist_layout(e.block_size, &grid, &lds);
+    int ldsh = e.hist_layout(e.launch_block(), &grid, &lds);
     if (!hist) {
         ldsh = 0;
         lds = 0;
@@ -1456,7 +1480,7 @@ static int launch_turn_t(const Engine &e, T *x, T *de, const T *rf, const T *acc
                                    : pick_turn<T, 2>(imode, hist, ldsh, publish, nt);
     int rc = lds_attribute((const void *)fn, lds);
     if (rc) return rc;
-    launch(fn, dim3(grid), dim3(e.block_size), lds, s, ev, x, de, e.n, a);
+    launch(fn, dim3(grid), dim3(e.launch_block()), lds, s, ev, x, de, e.n, a);
     return blmi_check_launch("turn");
 }
 
@@ -1493,7 +1517,7 @@ static int launch_turns_t(const Engine &e, T *x, T *de, const T *rf, const T *ac
     a.pending = e.d_base + 1;
     int grid = 0;
     size_t lds = 0;
-    const int ldsh = e.hist_layout(e.block_size, &grid, &lds);
+    const int ldsh = e.hist_layout(e.launch_block(), &grid, &lds);
     if (ldsh > 1) return blmi_set_error(BLMI_ERR_ARG, "multi-turn launch with u16 histogram rows");
     if (turns > kTurnBlockMax) return blmi_set_error(BLMI_ERR_ARG, "multi-turn launch of %d turns", turns);
     // the histogram words (mode 1), then the turns' programs
@@ -1503,7 +1527,7 @@ static int launch_turns_t(const Engine &e, T *x, T *de, const T *rf, const T *ac
                                     : pick_turns<T, 2>(ldsh);
     int rc = lds_attribute((const void *)fn, lds);
     if (rc) return rc;
-    launch(fn, dim3(grid), dim3(e.block_size), lds, s, ev, x, de, e.n, a, turns);
+    launch(fn, dim3(grid), dim3(e.launch_block()), lds, s, ev, x, de, e.n, a, turns);
     return blmi_check_launch("turns");
 }
 
@@ -1513,7 +1537,7 @@ bool Engine::multi_turn_ok() const {
     if (n_slices <= 0 || !d_counts) return false;
     int grid = 0;
     size_t lds = 0;
-    return hist_layout(block_size, &grid, &lds) <= 1;
+    return hist_layout(launch_block(), &grid, &lds) <= 1;
 }
 
 int Engine::multi_turn_piece(int left) const {
@@ -1558,7 +1582,7 @@ InducedArgs Engine::induced_args(int off) const {
     if (part_perm(&ps, &pl, &m1lo)) {
         int grid = 0;
         size_t lds = 0;
-        (void)hist_layout(block_size, &grid, &lds);
+        (void)hist_layout(launch_block(), &grid, &lds);
         ia.part = d_partials;
         ia.part_rows = grid;
         ia.part_lshift = pl;
@@ -1699,7 +1723,7 @@ int Engine::ensure_stats() {
     if (!stats_on) return BLMI_OK;
     int grid = 0;
     size_t lds = 0;
-    hist_layout(block_size, &grid, &lds);
+    hist_layout(launch_block(), &grid, &lds);
     if (grid == stats_grid && d_stats) return BLMI_OK;
     (void)hipFree(d_stats);
     d_stats = nullptr;
