@@ -129,15 +129,20 @@ __device__ __forceinline__ double cephes_sin(double x) {
 }
 
 // cephes_sin with one polynomial a lane, for kernels that keep the
-// coefficient table in LDS (kCephesTabDoubles doubles, 16-byte aligned:
-// kS0..kS5 of the sine branch, then kC0..kC5 of the cosine branch;
-// cephes_tab_fill writes it).  The lane's octant picks its branch's six
-// coefficients, evaluated in cephes_reduce's Horner order; the branch's last
-// steps, r + (r zz) P and (1 - zz/2) + (zz zz) P, become one A + B P with
-// A and B selected.  Every operation is one cephes_sin performs on the same
-// operands, so the result is bit-identical, and no lane evaluates the
-// polynomial its octant discards.
-constexpr int kCephesTabDoubles = 12;
+// coefficient table in LDS (kCephesTabDoubles doubles, 16-byte aligned, filled
+// by cephes_tab_fill): per branch the six Horner coefficients, then A0 and A1.
+// The lane's octant picks its branch's eight entries.  With w = r (sine) or zz
+// (cosine) the branch's last steps, r + (r zz) P and (1 - zz/2) + (zz zz) P,
+// are one A + B P with A = A0 + A1 w (0 + 1 r, or 1 + (-1/2) zz: both products
+// are exact) and B = w zz.  Every rounded operation is one cephes_sin performs
+// on the same operands, so the result is bit-identical but for the sign of a
+// zero result: the sign is the octant's xor x's sign bit, where cephes_sin
+// tests x < 0 (x = -0.0 gives -0.0 here).  The octant's bit 1, spread over a
+// word, is both the table offset's mask and the select of w.
+// 41 vector instructions a macroparticle-turn with the kick and drift around
+// it; with compares, four selected words more and a sign from two compares it
+// was 49 (25 plain turns of 1e6 macroparticles: 51.4 us a launch, now 46.5).
+constexpr int kCephesTabDoubles = 16;
 using LdsConstDoublePtr = __attribute__((address_space(3))) const double *;
 using LdsDoublePtr = __attribute__((address_space(3))) double *;
 
@@ -151,12 +156,16 @@ __device__ __forceinline__ double cephes_coef(int i) {
         case 3: return CephesD::kS3;
         case 4: return CephesD::kS4;
         case 5: return CephesD::kS5;
-        case 6: return CephesD::kC0;
-        case 7: return CephesD::kC1;
-        case 8: return CephesD::kC2;
-        case 9: return CephesD::kC3;
-        case 10: return CephesD::kC4;
-        default: return CephesD::kC5;
+        case 6: return 0.0;
+        case 7: return 1.0;
+        case 8: return CephesD::kC0;
+        case 9: return CephesD::kC1;
+        case 10: return CephesD::kC2;
+        case 11: return CephesD::kC3;
+        case 12: return CephesD::kC4;
+        case 13: return CephesD::kC5;
+        case 14: return 1.0;
+        default: return -0.5;
     }
 }
 
@@ -172,23 +181,25 @@ __device__ __forceinline__ double cephes_sin_tab(double x, LdsConstDoublePtr tab
     const double y = (double)j;
     const double r = ((ax - y * CephesD::kDP1) - y * CephesD::kDP2) - y * CephesD::kDP3;
     const double zz = r * r;
-    const bool cosb = cephes_cos_branch(j);
+    // all ones for the cosine branch (cephes_cos_branch), else zero
+    const int cosm = (int)((unsigned)j << 30) >> 31;
     using D2 = double __attribute__((ext_vector_type(2)));
     using LdsD2 = __attribute__((address_space(3))) const D2 *;
-    const LdsD2 c = reinterpret_cast<LdsD2>(tab + (cosb ? 6 : 0));
-    const D2 c01 = c[0], c23 = c[1], c45 = c[2];
+    const LdsD2 c = reinterpret_cast<LdsD2>(tab) + (cosm & 4);
+    const D2 c01 = c[0], c23 = c[1], c45 = c[2], ca = c[3];
     double p = c01.x;
     p = p * zz; p = p + c01.y;
     p = p * zz; p = p + c23.x;
     p = p * zz; p = p + c23.y;
     p = p * zz; p = p + c45.x;
     p = p * zz; p = p + c45.y;
-    const double A = cosb ? 1.0 - zz * 0.5 : r;
-    const double B = (cosb ? zz : r) * zz;
+    const double w = __hiloint2double((cosm & __double2hiint(zz)) | (~cosm & __double2hiint(r)),
+                                      (cosm & __double2loint(zz)) | (~cosm & __double2loint(r)));
+    const double A = ca.x + ca.y * w;
+    const double B = w * zz;
     const double out = A + B * p;
-    const unsigned flip = ((unsigned)j << 29) ^ (x < 0.0 ? 0x80000000u : 0u);
-    return __hiloint2double(__double2hiint(out) ^ (int)(flip & 0x80000000u),
-                            __double2loint(out));
+    const int sign = (int)((unsigned)j << 29) ^ __double2hiint(x);
+    return __hiloint2double(__double2hiint(out) ^ (sign & (int)0x80000000u), __double2loint(out));
 }
 
 // Both functions from one reduction (the adjoint needs the cosine).
@@ -254,10 +265,10 @@ __device__ __forceinline__ float cephes_sinf(float x) {
     const float c = ((2.443315711809948E-005f * z - 1.388731625493765E-003f) * z +
                      4.166664568298827E-002f) * z * z - 0.5f * z + 1.0f;
     const float out = cephes_cos_branch(j) ? c : s;
-    // the two sign changes (octant, then x < 0) as one: they cancel when
-    // both apply
-    const bool neg = ((j & 4) != 0) != (x < 0.0f);
-    return neg ? -out : out;
+    // the two sign changes (octant, then x < 0) as one flip of the sign bit;
+    // x's own sign bit stands for x < 0 (x = -0.0 gives -0.0)
+    const int sign = (int)((unsigned)j << 29) ^ __float_as_int(x);
+    return __int_as_float(__float_as_int(out) ^ (sign & (int)0x80000000u));
 }
 
 template <typename T> struct Trig;

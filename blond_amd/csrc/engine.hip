@@ -575,13 +575,20 @@ __global__ void __launch_bounds__(1024) turns_kernel(T *__restrict__ dt, T *__re
                 p.dc = a.drift[t + 1];
                 progs[k] = p;
             }
-            __syncthreads();
         }
+        // unit: charge 1 and no acceleration in any of the launch's turns (a
+        // coasting ring's protons, the common case): 1 s + 0 is s (but for the
+        // sign of a zero), two operations of a macroparticle-turn less
+        bool plain = q_charge == T(1);
+        if constexpr (NRF >= 0)
+            for (int k = threadIdx.x; k < K; k += blockDim.x) plain = plain && progs[k].acc == T(0);
+        const bool unit = __syncthreads_and(plain);
         // turns t0 .. tl-1 of M particles in lock step: M independent chains
         // of dependent FP64 operations keep the vector pipeline busy; the sum
         // is RfProg::kick_n's, in the same order
-        auto run = [&](T *x, T *e, auto m) {
+        auto run = [&](T *x, T *e, auto m, auto un) {
             constexpr int M = decltype(m)::value;
+            constexpr bool UNIT = decltype(un)::value;
             if constexpr (NRF >= 0) {
                 for (int k = 0; k < K; ++k) {
                     const TurnProg p = progs[k];
@@ -589,9 +596,11 @@ __global__ void __launch_bounds__(1024) turns_kernel(T *__restrict__ dt, T *__re
                     for (int j = 0; j < M; ++j) {
                         T s = T(0);
 #pragma unroll
-                        for (int r = 0; r < NRF; ++r)
-                            s = s + p.V[r] * TrigTab<T>::sin(p.w[r] * x[j] + p.phi[r], stab);
-                        e[j] = e[j] + (q_charge * s + p.acc);
+                        for (int r = 0; r < NRF; ++r) {
+                            const T v = p.V[r] * TrigTab<T>::sin(p.w[r] * x[j] + p.phi[r], stab);
+                            s = r == 0 ? v : s + v;
+                        }
+                        e[j] = e[j] + (UNIT ? s : q_charge * s + p.acc);
                         x[j] = x[j] + e_drift(p.dc, e[j], SOLVER);
                     }
                 }
@@ -609,33 +618,42 @@ __global__ void __launch_bounds__(1024) turns_kernel(T *__restrict__ dt, T *__re
                 }
             }
         };
-        // two pairs a thread at a time, i and i + stride (past the end the
-        // second slot repeats pair i, computed again and neither stored nor
-        // counted)
-        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n2; i += 2 * stride) {
-            const bool two = i + stride < n2;
-            const int64_t j = two ? i + stride : i;
-            const V2 xa = reinterpret_cast<const V2 *>(dt)[i], ea = reinterpret_cast<const V2 *>(dE)[i];
-            const V2 xb = reinterpret_cast<const V2 *>(dt)[j], eb = reinterpret_cast<const V2 *>(dE)[j];
-            T x[4] = {xa.x, xa.y, xb.x, xb.y}, e[4] = {ea.x, ea.y, eb.x, eb.y};
-            run(x, e, std::integral_constant<int, 4>{});
-            reinterpret_cast<V2 *>(dt)[i] = V2{x[0], x[1]};
-            reinterpret_cast<V2 *>(dE)[i] = V2{e[0], e[1]};
-            if (two) {
-                reinterpret_cast<V2 *>(dt)[j] = V2{x[2], x[3]};
-                reinterpret_cast<V2 *>(dE)[j] = V2{e[2], e[3]};
+        auto all = [&](auto un) {
+            // two pairs a thread at a time, i and i + stride (past the end the
+            // second slot repeats pair i, computed again and neither stored nor
+            // counted)
+            for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n2;
+                 i += 2 * stride) {
+                const bool two = i + stride < n2;
+                const int64_t j = two ? i + stride : i;
+                const V2 xa = reinterpret_cast<const V2 *>(dt)[i],
+                         ea = reinterpret_cast<const V2 *>(dE)[i];
+                const V2 xb = reinterpret_cast<const V2 *>(dt)[j],
+                         eb = reinterpret_cast<const V2 *>(dE)[j];
+                T x[4] = {xa.x, xa.y, xb.x, xb.y}, e[4] = {ea.x, ea.y, eb.x, eb.y};
+                run(x, e, std::integral_constant<int, 4>{}, un);
+                reinterpret_cast<V2 *>(dt)[i] = V2{x[0], x[1]};
+                reinterpret_cast<V2 *>(dE)[i] = V2{e[0], e[1]};
+                if (two) {
+                    reinterpret_cast<V2 *>(dt)[j] = V2{x[2], x[3]};
+                    reinterpret_cast<V2 *>(dE)[j] = V2{e[2], e[3]};
+                }
+                count(bin_of(x[0]));
+                count(bin_of(x[1]));
+                count(two ? bin_of(x[2]) : -1);
+                count(two ? bin_of(x[3]) : -1);
             }
-            count(bin_of(x[0]));
-            count(bin_of(x[1]));
-            count(two ? bin_of(x[2]) : -1);
-            count(two ? bin_of(x[3]) : -1);
-        }
+        };
+        if (NRF >= 0 && unit)
+            all(std::integral_constant<bool, NRF >= 0>{});
+        else
+            all(std::false_type{});
         if ((n & 1) && blockIdx.x == gridDim.x - 1 && threadIdx.x < 64) {
             // odd tail: lane 0 of the last block's first wavefront owns it
             int b = -1;
             if (threadIdx.x == 0) {
                 T x[1] = {dt[n - 1]}, e[1] = {dE[n - 1]};
-                run(x, e, std::integral_constant<int, 1>{});
+                run(x, e, std::integral_constant<int, 1>{}, std::false_type{});
                 dt[n - 1] = x[0];
                 dE[n - 1] = e[0];
                 b = bin_of(x[0]);

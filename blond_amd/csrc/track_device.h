@@ -82,7 +82,7 @@ struct RfProg {
         }
     }
     // kick_n with the sines of cephes_sin_tab (coefficients in LDS):
-    // bit-identical, about 13 fewer FP64 operations a sine
+    // bit-identical up to the sign of zeros
     template <int NRF>
     __device__ __forceinline__ T kick_tab(T t, T charge, T acc, LdsConstDoublePtr tab) const {
         static_assert(NRF <= kRfRegs, "NRF exceeds the systems held in registers");
@@ -94,9 +94,13 @@ struct RfProg {
             for (int j = kRfRegs; j < n; ++j) s = s + Vt[j] * TrigTab<T>::sin(wt[j] * t + pt[j], tab);
             return charge * s + acc;
         } else {
+            // 0 + the first term is that term (but for the sign of a zero)
             T s = T(0);
 #pragma unroll
-            for (int j = 0; j < NRF; ++j) s = s + V[j] * TrigTab<T>::sin(w[j] * t + phi[j], tab);
+            for (int j = 0; j < NRF; ++j) {
+                const T v = V[j] * TrigTab<T>::sin(w[j] * t + phi[j], tab);
+                s = j == 0 ? v : s + v;
+            }
             return charge * s + acc;
         }
     }
