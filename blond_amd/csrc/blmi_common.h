@@ -314,6 +314,13 @@ __device__ __forceinline__ double2 interp_entry(double v0, double v1, double bcb
     return make_double2(k, (charge * v0 - bcb * k) + 0.0);
 }
 
+// Bin centre b of uniform bins from cut_left in steps of `step`: the mean of the
+// edges b step + cut_left and (b + 1) step + cut_left, rounded as numpy's
+// linspace and (edges[:-1] + edges[1:]) / 2 round them.
+__device__ __forceinline__ double bin_line(double b, double cut_left, double step) {
+    return ((b * step + cut_left) + ((b + 1.0) * step + cut_left)) * 0.5;
+}
+
 // A table entry as stored: a (slope, intercept) pair of doubles, or with f32
 // of floats, which hold the single build's FP32 values exactly and halve the
 // bytes the kick gathers (the table then holds float2 entries; its

@@ -86,8 +86,14 @@ struct TurnArgs {
     int win_lo, win_bins;
     unsigned *cnt_out;
     // interpolation table from L2: entries [tw_lo, tw_lo + tw_n) staged in
-    // LDS after the histogram (tw_n 0: none)
+    // LDS after the histogram (tw_n 0: none); FP64 NEAR kernels stage the
+    // tw_n + 1 voltages under them, and form an entry from two of them and the
+    // bin centre on a line of spacing `step` from the left cut, unless a word
+    // of bc_off says that the bin centres are not on it
     int tw_lo, tw_n;
+    const double *volt;
+    double step;
+    const int *bc_off;                 // [kWave]
     // bunch moments of the coordinates after the drift: workgroup b writes
     // sum(dt - shift_t), sum((dt - shift_t)^2), sum(dE - shift_e),
     // sum((dE - shift_e)^2) of its particles to stats[(t + 1) * grid + b]
@@ -210,11 +216,62 @@ using GlobalPtr = __attribute__((address_space(1))) V *;
 template <typename T> struct TabEntry { using type = double2; };
 template <> struct TabEntry<float> { using type = float2; };
 
+// bc_off[b] = 1 where a bin centre of workgroup b's share (grid: kWave) is not
+// the middle of the edges b step + cut_left and (b + 1) step + cut_left, as
+// numpy's linspace and mean give them
+__global__ void __launch_bounds__(1024) bin_line_kernel(const double *__restrict__ bc, int n_tab,
+                                                        double cut_left, double step,
+                                                        int *__restrict__ bc_off) {
+    int off = 0;
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < n_tab; b += gridDim.x * blockDim.x)
+        off |= bc[b] != bin_line(b, cut_left, step);
+    off = __syncthreads_or(off);
+    if (threadIdx.x == 0) bc_off[blockIdx.x] = off;
+}
+
+// 16 (double) or 8 (float) bytes of a pair of coordinates through a buffer
+// descriptor: an offset past its end loads zeros and stores nothing
+template <typename V2, int POLICY>
+__device__ __forceinline__ V2 buffer_load_pair(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    if constexpr (sizeof(V2) == 16)
+        return __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, POLICY));
+    else
+        return __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, POLICY));
+}
+template <typename V2, int POLICY>
+__device__ __forceinline__ void buffer_store_pair(__amdgpu_buffer_rsrc_t r, unsigned off, V2 v) {
+    if constexpr (sizeof(V2) == 16) {
+        using W = unsigned __attribute__((ext_vector_type(4)));
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(W, v), r, (int)off, 0, POLICY);
+    } else {
+        using W = unsigned __attribute__((ext_vector_type(2)));
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(W, v), r, (int)off, 0, POLICY);
+    }
+}
+constexpr int kPolicyNt = 2;  // the non-temporal bit of a buffer access
+// word 3 of a raw buffer's descriptor (32-bit data format)
+constexpr int kBufferFlags = 0x00027000;
+
 // NT: the coordinates are read and written with non-temporal loads and
 // stores (for bunches larger than the last-level cache, where they stream
 // from HBM either way and, kept out of the caches' recently-used lines,
 // leave L2 to the interpolation table's gathers)
-template <typename T, int SOLVER, int INTERP, bool HIST, int LDSH, bool PUBLISH, bool NT = false>
+//
+// NEAR (the u16-row kernels, coordinates within 32-bit byte offsets, no merged
+// count): the pairs go through buffer descriptors, whose range check stands
+// for the clamped loads, the sink and the 64-bit addresses, and no constant is
+// moved into vector registers.  That leaves room in the FP64 kernel for the
+// voltage window: 8 bytes a bin in LDS and not 16, so twice as many bins (12032
+// at 65536 slices; 64 % and not 35 % of a bunch of 6560 bins rms), each entry
+// formed from two voltages with 12 operations more.  A macroparticle outside
+// the window gathers a 128-byte line for its 16 bytes from L2, beside the
+// stream of the coordinates.  Two RF systems, 65536 slices, kernel: 1e7
+// macroparticles 67.6 -> 66.5 us, 3e7 295 -> 241 us (the stream alone at the
+// rate of an in-place copy: 41 and 175 us); FP32, addresses only, 1e7 45.9 ->
+// 44.5 us.  Measured the same: two pairs more in flight, gathers issued before
+// the stores, part of a 3e7 bunch kept in the last-level cache.
+template <typename T, int SOLVER, int INTERP, bool HIST, int LDSH, bool PUBLISH, bool NT = false,
+          bool NEAR = false>
 __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__restrict__ dE,
                                                     int64_t n, TurnArgs<T> a) {
     using V2 = typename Vec2<T>::type;
@@ -275,6 +332,8 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         xa = reinterpret_cast<const V2 *>(dt)[clamp(i_first)];
         ea = reinterpret_cast<const V2 *>(dE)[clamp(i_first)];
     }
+    constexpr bool kVoltWindow = NEAR && sizeof(T) == 8;
+    const bool line_off = kVoltWindow && __any(a.bc_off[threadIdx.x % kWave]);
     // the histogram words (with windowed rows, the window's); the padded
     // layout adds one word per 2^part_shift (none when 31)
     const int hwords = (HIST && LDSH) ? ((LDSH == 2 && a.win_bins) ? a.win_bins / 2
@@ -293,7 +352,11 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         if (INTERP == 2)
             for (int k = threadIdx.x; k < a.n_tab; k += blockDim.x) ltab[k] = gtab[k];
         if (tw_on)
-            for (int k = threadIdx.x; k < a.tw_n; k += blockDim.x) ltab[k] = gtab[a.tw_lo + k];
+            if constexpr (kVoltWindow)
+                for (int k = threadIdx.x; k <= a.tw_n; k += blockDim.x)
+                    reinterpret_cast<double *>(ltab)[k] = a.volt[a.tw_lo + k];
+            else
+                for (int k = threadIdx.x; k < a.tw_n; k += blockDim.x) ltab[k] = gtab[a.tw_lo + k];
     }
     __syncthreads();  // the LDS set-up, and the sine's coefficient table
     // the table window (lds_hist itself, never read, when there is none)
@@ -310,7 +373,8 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
     // v_readlane at every use)
     T q_charge = a.charge, q_acc = acc, q_cl = a.cut_left, q_ibw = a.inv_bw;
     T q_ntab = (T)a.n_tab, q_ns = (T)a.n_slices, q_bc0 = bc0, q_tibw = ibw;
-    int q_twlo = a.tw_lo, q_twn = a.tw_n, q_wlo = a.win_lo, q_wn = a.win_bins;
+    int q_twlo = a.tw_lo, q_twn = line_off ? 0 : a.tw_n, q_wlo = a.win_lo, q_wn = a.win_bins;
+    const T q_step = (T)a.step;
     uint64_t q_tabp = (uint64_t)a.tab, q_cntp = (uint64_t)a.cnt_out;
     auto pin_constants = [&]() {
         asm volatile("" : "+v"(q_charge), "+v"(q_acc), "+v"(q_cl), "+v"(q_ibw));
@@ -335,8 +399,12 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
                 TabE kg;
                 kg.x = kv.x;
                 kg.y = kv.y;
-                const TabE kl = ltw[intw ? kw : 0];
-                g.k = intw ? kl : kg;
+                if constexpr (kVoltWindow) {
+                    g.k = kg;  // finish() reads the window itself
+                } else {
+                    const TabE kl = ltw[intw ? kw : 0];
+                    g.k = intw ? kl : kg;
+                }
             } else {
                 g.k = INTERP == 2 ? ltab[fi] : gtab[fi];
             }
@@ -347,10 +415,28 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
     // keep the order e + interp + rf
     auto finish = [&](T &x, T &e, const Tab &g, auto nrf) -> int {
         constexpr int NRF = decltype(nrf)::value;
+        T v0 = T(0), v1 = T(0), f0 = T(0);
+        bool win = false;
+        if constexpr (kVoltWindow) {
+            f0 = floor((x - q_bc0) * q_tibw);
+            const int kw = (int)f0 - q_twlo;
+            win = g.in && (unsigned)kw < (unsigned)q_twn;
+            const double *lv = reinterpret_cast<const double *>(ltw) + (win ? kw : 0);
+            v0 = lv[0];
+            v1 = lv[1];
+        }
         const T rf = rfp.template kick_tab<NRF>(x, q_charge, q_acc, stab);
         if (INTERP) {
+            T slope = (T)g.k.x, cut = (T)g.k.y;
+            if constexpr (kVoltWindow) {
+                // interp_entry on the bin's line centre
+                const double2 k = interp_entry(v0, v1, bin_line(f0, q_cl, q_step), q_charge,
+                                               q_tibw, false);
+                slope = win ? k.x : slope;
+                cut = win ? k.y : cut;
+            }
             // a select, not a branch: nothing waits on the gather before the sines
-            const T ei = e + (x * (T)g.k.x + (T)g.k.y);
+            const T ei = e + (x * slope + cut);
             e = g.in ? ei : e;
         }
         e = e + rf;
@@ -378,7 +464,7 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
             // any window's width
             const int wb = bin - q_wlo;
             const bool in = (unsigned)wb < (unsigned)q_wn;
-            if (a.max_peel > 0)
+            if (!NEAR && a.max_peel > 0)
                 lds_count<true>(lds_hist, in ? wb : -1, a.max_peel, a.part_shift);
             else if (in)
                 lds_add1<true>(lds_hist, wb, a.part_shift);
@@ -386,36 +472,52 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
                 __hip_atomic_fetch_add(&reinterpret_cast<GlobalPtr<unsigned>>(q_cntp)[bin], 1u,
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else if (LDSH) {
-            lds_count<LDSH == 2>(lds_hist, bin, a.max_peel, a.part_shift);
+            lds_count<LDSH == 2>(lds_hist, bin, NEAR ? 0 : a.max_peel, a.part_shift);
         } else if (bin >= 0) {
             atomic_add_agent(&counts[bin], 1u);
         }
     };
+    // NEAR: descriptors of the whole pairs; a pair's byte offset runs along with
+    // its index
+    const int bytes = NEAR ? (int)(unsigned)(n2 * (int64_t)sizeof(V2)) : 0;
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc((void *)dt, 0, bytes, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t re =
+        __builtin_amdgcn_make_buffer_rsrc((void *)dE, 0, bytes, kBufferFlags);
+    constexpr int kPolicy = NT ? kPolicyNt : 0;
+    const unsigned stride_bytes = (unsigned)stride * (unsigned)sizeof(V2);
     // one copy of the particle loop per RF-system count (see with_rf_count)
     with_rf_count(a.n_rf, [&](auto nrf) {
-    rfp.template pin<decltype(nrf)::value>();
-    pin_constants();
+    if constexpr (!NEAR) {
+        rfp.template pin<decltype(nrf)::value>();
+        pin_constants();
+    }
     // one pair: RF kick, interpolated kick, drift, store, count; and (more)
     // the other slot's table loads and this slot's reload two pairs ahead
     V2 *const sink = reinterpret_cast<V2 *>(a.sink) + 2 * (threadIdx.x % kWave);
     auto pair = [&](auto more, V2 &x, V2 &e, Tab &g0, Tab &g1, const V2 &xo, Tab &go0,
-                    Tab &go1, int64_t i) {
-        const bool own = i < n2;
+                    Tab &go1, int64_t i, unsigned off) {
+        const bool own = NEAR ? off < (unsigned)bytes : i < n2;
         int b0 = finish(x.x, e.x, g0, nrf);
         int b1 = finish(x.y, e.y, g1, nrf);
-        // the target is chosen as an integer and hidden from the optimiser,
-        // which would otherwise split the store into two guarded stores:
-        // with a divergent branch around them the waits above lose count
-        uint64_t at = own ? (uint64_t)(reinterpret_cast<V2 *>(dt) + i) : (uint64_t)sink;
-        uint64_t ae = own ? (uint64_t)(reinterpret_cast<V2 *>(dE) + i) : (uint64_t)(sink + 1);
-        asm volatile("" : "+v"(at), "+v"(ae));
-        using NV2 = T __attribute__((ext_vector_type(2)));
-        if constexpr (NT) {
-            __builtin_nontemporal_store(NV2{x.x, x.y}, reinterpret_cast<GlobalPtr<NV2>>(at));
-            __builtin_nontemporal_store(NV2{e.x, e.y}, reinterpret_cast<GlobalPtr<NV2>>(ae));
+        if constexpr (NEAR) {
+            buffer_store_pair<V2, kPolicy>(rx, off, x);
+            buffer_store_pair<V2, kPolicy>(re, off, e);
         } else {
-            *reinterpret_cast<GlobalPtr<NV2>>(at) = NV2{x.x, x.y};
-            *reinterpret_cast<GlobalPtr<NV2>>(ae) = NV2{e.x, e.y};
+            // the target is chosen as an integer and hidden from the optimiser,
+            // which would otherwise split the store into two guarded stores:
+            // with a divergent branch around them the waits above lose count
+            uint64_t at = own ? (uint64_t)(reinterpret_cast<V2 *>(dt) + i) : (uint64_t)sink;
+            uint64_t ae = own ? (uint64_t)(reinterpret_cast<V2 *>(dE) + i) : (uint64_t)(sink + 1);
+            asm volatile("" : "+v"(at), "+v"(ae));
+            using NV2 = T __attribute__((ext_vector_type(2)));
+            if constexpr (NT) {
+                __builtin_nontemporal_store(NV2{x.x, x.y}, reinterpret_cast<GlobalPtr<NV2>>(at));
+                __builtin_nontemporal_store(NV2{e.x, e.y}, reinterpret_cast<GlobalPtr<NV2>>(ae));
+            } else {
+                *reinterpret_cast<GlobalPtr<NV2>>(at) = NV2{x.x, x.y};
+                *reinterpret_cast<GlobalPtr<NV2>>(ae) = NV2{e.x, e.y};
+            }
         }
         if (own) {
             if (a.stats) {
@@ -428,8 +530,12 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         if constexpr (decltype(more)::value) {
             go0 = gather(xo.x);
             go1 = gather(xo.y);
-            const int64_t j = clamp(i + 2 * stride);
-            if constexpr (NT) {
+            if constexpr (NEAR) {
+                x = buffer_load_pair<V2, kPolicy>(rx, off + 2 * stride_bytes);
+                e = buffer_load_pair<V2, kPolicy>(re, off + 2 * stride_bytes);
+            } else if constexpr (NT) {
+                const int64_t j = clamp(i + 2 * stride);
+                using NV2 = T __attribute__((ext_vector_type(2)));
                 const NV2 xv =
                     __builtin_nontemporal_load(reinterpret_cast<GlobalPtr<const NV2>>((uint64_t)dt) + j);
                 const NV2 ev =
@@ -437,6 +543,7 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
                 x = V2{xv.x, xv.y};
                 e = V2{ev.x, ev.y};
             } else {
+                const int64_t j = clamp(i + 2 * stride);
                 x = reinterpret_cast<const V2 *>(dt)[j];
                 e = reinterpret_cast<const V2 *>(dE)[j];
             }
@@ -452,12 +559,14 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         // would again leave the waits conservative); an odd count's last pair
         // after the loop
         constexpr std::true_type more{};
+        unsigned off = (unsigned)i_first * (unsigned)sizeof(V2);
         for (int64_t k = 0; k + 1 < iters; k += 2) {
-            pair(more, xa, ea, ga0, ga1, xb, gb0, gb1, i_first + k * stride);
-            pair(more, xb, eb, gb0, gb1, xa, ga0, ga1, i_first + (k + 1) * stride);
+            pair(more, xa, ea, ga0, ga1, xb, gb0, gb1, i_first + k * stride, off);
+            pair(more, xb, eb, gb0, gb1, xa, ga0, ga1, i_first + (k + 1) * stride, off + stride_bytes);
+            off += 2 * stride_bytes;
         }
         if (iters & 1)
-            pair(std::false_type{}, xa, ea, ga0, ga1, xb, gb0, gb1, i_first + (iters - 1) * stride);
+            pair(std::false_type{}, xa, ea, ga0, ga1, xb, gb0, gb1, i_first + (iters - 1) * stride, off);
     }
     if ((n & 1) && blockIdx.x == gridDim.x - 1 && threadIdx.x < 64) {
         // odd tail: the first wavefront of the last block takes part in the
@@ -762,7 +871,9 @@ void Engine::release() {
     (void)hipFree(d_drift);
     (void)hipFree(d_base);
     (void)hipFree(d_sink);
+    (void)hipFree(d_bc_off);
     d_sink = nullptr;
+    d_bc_off = nullptr;
     (void)hipFree(d_counts);
     (void)hipFree(d_table);
     (void)hipFree(d_Z);
@@ -1118,6 +1229,35 @@ int Engine::launch_block() const {
     return b;
 }
 
+// The u16-row intensity kernels take buffer descriptors (turn_kernel NEAR)
+// while every offset of a launch, two strides past the end included, fits 32
+// bits, the counts are not merged and the table is the induced voltage's own.
+bool Engine::near_kernel(int imode, bool hist, int ldsh) const {
+    if (imode != 1 || !hist || ldsh != 2 || !intensity || interp_rf || max_peel > 0) return false;
+    int grid = 0;
+    size_t lds = 0;
+    const int block = launch_block();
+    (void)hist_layout(block, &grid, &lds);
+    const int64_t pair = f32 ? 2 * sizeof(float) : 2 * sizeof(double);
+    return (n / 2 + 4 * (int64_t)grid * block) * pair < (int64_t)1 << 32;
+}
+
+// Words of bc_off for the voltage window, from the bin centres as they are now.
+int Engine::check_bin_line(hipStream_t s) {
+    if (f32 || !intensity || ordered() || n_slices < 2) return BLMI_OK;
+    int grid = 0;
+    size_t lds = 0;
+    const int mode = hist_layout(launch_block(), &grid, &lds);
+    if (mode != 2 || !near_kernel(1, d_counts != nullptr, mode)) return BLMI_OK;
+    if (!d_bc_off) {
+        invalidate_graph();
+        BLMI_HIP_TRY(hipMalloc(&d_bc_off, sizeof(int) * kWave));
+    }
+    hipLaunchKernelGGL(bin_line_kernel, dim3(kWave), dim3(1024), 0, s, bc, n_slices - 1, cut_left,
+                       bin_step(), d_bc_off);
+    return blmi_check_launch("bin_line");
+}
+
 int Engine::hist_layout(int block, int *grid_out, size_t *lds_out) const {
     int grid = device_cu_count() * blocks_per_cu;
     const int64_t n2 = n / 2;
@@ -1368,7 +1508,10 @@ template <typename T>
 using TurnFn = void (*)(T *, T *, int64_t, TurnArgs<T>);
 
 template <typename T, int S>
-static TurnFn<T> pick_turn(int interp, bool hist, int ldsh, bool publish, bool nt) {
+static TurnFn<T> pick_turn(int interp, bool hist, int ldsh, bool publish, bool nt, bool near) {
+    if (near)
+        return nt ? turn_kernel<T, S, 1, true, 2, false, true, true>
+                  : turn_kernel<T, S, 1, true, 2, false, false, true>;
     // publish: plain turns (no intensity effects), whose histogram is the
     // caller's profile; with intensity effects the induced-voltage launch
     // consumes the counts instead
@@ -1472,30 +1615,40 @@ static int launch_turn_t(const Engine &e, T *x, T *de, const T *rf, const T *acc
         imode = 2;
         lds = hist_bytes + tab_bytes;
     }
+    const bool publish = !e.intensity;
+    const bool near = e.near_kernel(imode, hist, ldsh);
+    if (near) {
+        a.volt = e.volt;
+        a.step = e.bin_step();
+        a.bc_off = e.d_bc_off;
+    }
     if (imode == 1 && hist && ldsh == 2 && a.n_tab > 0) {
         // the LDS the u16 rows leave holds a window of the table, centred on
         // the rows' window (else on the slice range)
         const size_t base = (lds + 15) / 16 * 16;
         const size_t cap = (size_t)device_max_lds();
         const size_t avail = cap > base + kStaticLdsMargin ? cap - base - kStaticLdsMargin : 0;
-        int tw = (int)std::min<size_t>(avail / entry, (size_t)a.n_tab) & ~63;
+        // FP64 NEAR kernels: voltages, one more than the entries they give
+        const bool volts = near && !e.f32;
+        const size_t word = volts ? sizeof(double) : entry;
+        const size_t fit = avail / word - (volts && avail >= word ? 1 : 0);
+        int tw = (int)std::min<size_t>(fit, (size_t)a.n_tab) & ~63;
         if (tw >= 256) {
             const int c = a.win_bins ? a.win_lo + a.win_bins / 2 : a.n_tab / 2;
             int lo = c - tw / 2;
             lo = std::max(0, std::min(lo, a.n_tab - tw));
             a.tw_lo = lo;
             a.tw_n = tw;
-            lds = base + entry * (size_t)tw;
+            lds = base + word * (size_t)(tw + (volts ? 1 : 0));
         }
     }
-    const bool publish = !e.intensity;
     // non-temporal coordinates when they exceed the last-level cache (c3 at
     // 3e7 macroparticles, 480 MB: particle kernel 319 -> 285 us; at 1e7,
     // cache-resident, they would cost 68 -> 99 us)
     const bool nt = (double)sizeof(T) * 2.0 * (double)e.n > kLastLevelCacheBytes;
-    TurnFn<T> fn = e.solver == 0   ? pick_turn<T, 0>(imode, hist, ldsh, publish, nt)
-                   : e.solver == 1 ? pick_turn<T, 1>(imode, hist, ldsh, publish, nt)
-                                   : pick_turn<T, 2>(imode, hist, ldsh, publish, nt);
+    TurnFn<T> fn = e.solver == 0   ? pick_turn<T, 0>(imode, hist, ldsh, publish, nt, near)
+                   : e.solver == 1 ? pick_turn<T, 1>(imode, hist, ldsh, publish, nt, near)
+                                   : pick_turn<T, 2>(imode, hist, ldsh, publish, nt, near);
     int rc = lds_attribute((const void *)fn, lds);
     if (rc) return rc;
     launch(fn, dim3(grid), dim3(e.launch_block()), lds, s, ev, x, de, e.n, a);
@@ -2050,6 +2203,8 @@ int Engine::time_kernels(int turns, hipStream_t user, float *ms_induced, float *
         prc = launch_mtw_load(d_base, d_mem, d_mem + n_mem, n_mem, mem_user, own_stream);
         if (prc) return prc;
     }
+    prc = check_bin_line(own_stream);
+    if (prc) return prc;
     std::vector<hipEvent_t> ev(4 * (size_t)turns, nullptr);
     for (auto &x : ev) BLMI_HIP_TRY(hipEventCreate(&x));
     int rc = BLMI_OK;
@@ -2122,6 +2277,8 @@ int Engine::track(int turns, hipStream_t user, bool use_graph) {
         prc = launch_mtw_load(d_base, d_mem, d_mem + n_mem, n_mem, mem_user, own_stream);
         if (prc) return prc;
     }
+    prc = check_bin_line(own_stream);
+    if (prc) return prc;
     int done = 0;
     int rc = BLMI_OK;
     if (use_graph && turns >= chunk) {

@@ -1,0 +1,63 @@
+"""The u16-row particle kernel with buffer descriptors and the voltage window:
+the same bits as the kernel it stands in for (which merged counts still take),
+and the gathered table where the bin centres are not on the cuts' line."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+if not torch.cuda.is_available():  # pragma: no cover
+    pytest.skip("no GPU", allow_module_level=True)
+
+from blond_amd.utils import bm  # noqa: E402
+from blond_amd.workloads import build_workload  # noqa: E402
+
+
+def _run(name, turns, peel, **kw):
+    w = build_workload(name, n_turns=turns + 1, **kw)
+    w.fused(1, max_peel=peel)
+    w.fused(turns - 1)
+    return [a.cpu().numpy() for a in (w.beam.dt, w.beam.dE, w.profile.n_macroparticles,
+                                      w.tiv.induced_voltage)]
+
+
+# u16 rows without a histogram window, with one, and a slice count whose
+# transform is no power of two; one and two RF systems; odd and tiny bunches,
+# an odd and an even number of pairs a thread
+@pytest.mark.parametrize("name,n_slices,n_fft", [("c2", 20000, 20000), ("c2", 32768, 65536),
+                                                 ("c3", 65536, 131072), ("c2", 40000, 48000)])
+@pytest.mark.parametrize("n", [1, 4097, 300001, 2 * 262144 + 2, 4 * 262144 + 3])
+@pytest.mark.parametrize("precision", ["double", "single"])
+def test_same_bits_as_the_gathering_kernel(name, n_slices, n_fft, n, precision):
+    bm.use_precision(precision)
+    try:
+        kw = dict(n_particles=n, n_slices=n_slices, n_fft=n_fft)
+        for a, b in zip(_run(name, 4, 0, **kw), _run(name, 4, 1, **kw)):
+            assert np.array_equal(a, b)
+    finally:
+        bm.use_precision("double")
+
+
+def _turn_matches_oracle(w):
+    ref = orc.track(w.oracle_copy(), 1)
+    w.fused(1)
+    assert np.array_equal(w.profile.n_macroparticles.cpu().numpy(), ref["profile"])
+    for got, want in ((w.beam.dt, ref["dt"]), (w.beam.dE, ref["dE"])):
+        assert np.abs(got.cpu().numpy() - want).max() <= 1e-12 * np.abs(want).max()
+
+
+def test_bin_centres_off_the_line_use_the_table():
+    """Centres moved by a tenth of a bin inside the window, before the first
+    turn and in place between two calls: the kick follows them."""
+    w = build_workload("c3", n_particles=200001, n_turns=6, n_slices=65536, n_fft=131072,
+                       intensity=1e13)
+    _turn_matches_oracle(w)
+    bc = w.profile.bin_centers
+    step = float(w.profile.bin_size)
+    for at in (32768, 31000):
+        bc[at:at + 1000] += 0.1 * step
+        _turn_matches_oracle(w)
+    bc[32768:33768] -= 0.1 * step
