@@ -776,15 +776,19 @@ __global__ void __launch_bounds__(1024) turns_kernel(T *__restrict__ dt, T *__re
     }
 }
 
-// Plain mode, end of a track() call: publish the last turn's counts (one
-// workgroup, so the pending flag is cleared after every bin is done).
-__global__ void publish_kernel(const int *base, int off, unsigned *counts0, unsigned *counts1,
-                               int groups, int *pending, double *profile, int n_slices) {
-    const int t = *base + off;  // histogram of dt_t
-    if (pending[t & 1] != t) return;
-    publish_range((t & 1) ? counts1 : counts0, profile, n_slices, groups, 0, n_slices);
+// Plain mode, end of a chunk: publish the last turn's counts (one workgroup,
+// so the pending flag is cleared after every bin is done) and, with `advance`,
+// move the turn base on (a launch of its own where other launches of the chunk
+// still read it: 4 us and a gap).
+__global__ void publish_kernel(int *base, int off, unsigned *counts0, unsigned *counts1, int groups,
+                               int *pending, double *profile, int n_slices, int advance) {
+    const int b = *base, t = b + off;  // histogram of dt_t
+    const bool held = pending[t & 1] == t;
+    if (held) publish_range((t & 1) ? counts1 : counts0, profile, n_slices, groups, 0, n_slices);
     __syncthreads();
-    if (threadIdx.x == 0) pending[t & 1] = -1;
+    if (threadIdx.x != 0) return;
+    if (held) pending[t & 1] = -1;
+    if (advance) *base = b + advance;
 }
 
 __global__ void to_float_kernel(const double *__restrict__ src, float *__restrict__ dst, int n) {
@@ -2145,10 +2149,14 @@ int Engine::launch_turns(hipStream_t s, int count, bool advance) {
 }
 
 int Engine::finish_chunk(hipStream_t s, int count) {
-    if (!intensity && n_slices > 0 && d_counts) {
+    // the publish launch also advances the turn base where nothing after it
+    // reads the old one (the moments' sum does)
+    const bool publish = !intensity && n_slices > 0 && d_counts;
+    const bool advanced = publish && !stats_on;
+    if (publish) {
         hipLaunchKernelGGL(publish_kernel, dim3(1), dim3(1024), 0, s, d_base, count, d_counts,
                            d_counts + (size_t)groups * n_slices, groups, d_base + 1, profile,
-                           n_slices);
+                           n_slices, advanced ? count : 0);
         int rc = blmi_check_launch("publish");
         if (rc) return rc;
     }
@@ -2167,9 +2175,11 @@ int Engine::finish_chunk(hipStream_t s, int count) {
         int rc = blmi_check_launch("moments_reduce");
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(1), 0, s, d_base, count);
-    int rc = blmi_check_launch("advance");
-    if (rc) return rc;
+    if (!advanced) {
+        hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(1), 0, s, d_base, count);
+        int rc = blmi_check_launch("advance");
+        if (rc) return rc;
+    }
     // the multi-turn memory of the new turn base, for the caller
     if (n_mem > 0 && mem_user)
         return launch_mtw_publish(d_base, d_mem, d_mem + n_mem, n_mem, mem_user, s);
