@@ -157,11 +157,19 @@ def last_error() -> str:
     return msg.decode() if msg else ""
 
 
-def call(name: str, *args) -> None:
-    """Call ``name`` and raise BlmiError on a non-zero status."""
+_FUNCTIONS: dict = {}
+
+
+def _function(name: str):
     lib = load()
     if name in lib.blmi_missing:
         raise LibraryNotAvailable(f"{name} is not in {LIB_PATH}: rebuild the library")
-    rc = getattr(lib, name)(*args)
+    fn = _FUNCTIONS[name] = getattr(lib, name)
+    return fn
+
+
+def call(name: str, *args) -> None:
+    """Call ``name`` and raise BlmiError on a non-zero status."""
+    rc = (_FUNCTIONS.get(name) or _function(name))(*args)
     if rc != 0:
         raise BlmiError(f"{name} failed ({rc}): {last_error()}")

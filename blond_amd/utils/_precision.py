@@ -13,6 +13,7 @@ class PrecisionClass:
         self.set(_precision)
 
     def set(self, _precision: str = "double"):
+        self._torch_dtype = None
         if _precision in ["single", "s", "32", "float32", "float", "f"]:
             self.str = "single"
             self.real_t = np.float32
@@ -30,9 +31,11 @@ class PrecisionClass:
 
     @property
     def torch_dtype(self):
-        import torch
+        if self._torch_dtype is None:
+            import torch
 
-        return torch.float64 if self.num == 2 else torch.float32
+            self._torch_dtype = torch.float64 if self.num == 2 else torch.float32
+        return self._torch_dtype
 
 
 precision = PrecisionClass("double")

@@ -37,21 +37,34 @@ from ._precision import precision
 _SOLVERS = {"simple": 0, "legacy": 1, "exact": 2}
 
 
+# A turn of a small bunch through these calls is bound by their host cost
+# (5e4 macroparticles, three calls and the moments: 87 us a turn
+# with a device query, a stream look-up by name and a ctypes
+# object per argument in every call; 72 us with what cannot change held here).
+_TORCH = None  # torch, once a GPU has been seen
+
+
 def _torch():
-    import torch
+    global _TORCH
+    if _TORCH is None:
+        import torch
 
-    if not torch.cuda.is_available():
-        raise _lib.LibraryNotAvailable(
-            "blond_amd needs a ROCm GPU: torch.cuda.is_available() is False")
-    return torch
+        if not torch.cuda.is_available():
+            raise _lib.LibraryNotAvailable(
+                "blond_amd needs a ROCm GPU: torch.cuda.is_available() is False")
+        _TORCH = torch
+    return _TORCH
 
 
-def _stream(torch) -> ct.c_void_p:
-    return ct.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream(torch) -> int:
+    """The current device's current stream (its handle; 0 is the default)."""
+    return torch.cuda.current_stream(torch.cuda.current_device()).cuda_stream
 
 
 class _Staged:
     """Device view of one argument; writes numpy in/out arrays back on exit."""
+
+    __slots__ = ("torch", "src", "writeback", "dev", "ptr")
 
     def __init__(self, torch, arr: Any, writeback: bool, dtype=None, name: str = "array"):
         self.torch = torch
@@ -74,10 +87,7 @@ class _Staged:
                 assert a.dtype == np.dtype(precision.real_t), f"{name}: dtype {a.dtype} != {precision.real_t}"
             host = np.ascontiguousarray(a, dtype=precision.real_t if dtype is None else _np_of(dt))
             self.dev = torch.from_numpy(host).to("cuda")
-
-    @property
-    def ptr(self) -> ct.c_void_p:
-        return ct.c_void_p(self.dev.data_ptr())
+        self.ptr = self.dev.data_ptr()
 
     def finish(self):
         if self.writeback:
@@ -95,8 +105,8 @@ def _suffix() -> str:
     return "" if precision.num == 2 else "_f32"
 
 
-def _real(x) -> Any:
-    return precision.c_real_t(float(x))
+# a scalar argument: the bound signatures convert to double or float
+_real = float
 
 
 def _len(a) -> int:
@@ -399,11 +409,10 @@ def beam_statistics(dt, dE, id=None):
         ids = ids.to(torch.int64).contiguous()
     out = torch.empty(5, dtype=torch.float64, device="cuda")
     name = "blmi_beam_statistics" + ("_f32" if x.dtype == torch.float32 else "")
-    _lib.call(name, ct.c_void_p(x.data_ptr()), ct.c_void_p(e.data_ptr()),
-              ct.c_void_p(ids.data_ptr()) if ids is not None else None, int(x.numel()),
-              ct.c_void_p(out.data_ptr()), _stream(torch))
-    r = out.cpu().numpy()
-    return int(r[0]), float(r[1]), float(r[2]), float(r[3]), float(r[4])
+    _lib.call(name, x.data_ptr(), e.data_ptr(), ids.data_ptr() if ids is not None else None,
+              int(x.numel()), out.data_ptr(), _stream(torch))
+    r = out.tolist()
+    return int(r[0]), *r[1:]
 
 
 def induced_voltage_1turn(profile, total_impedance, n_fft: int, scale: float, n_out: int = 0):
