@@ -130,16 +130,29 @@ __device__ __forceinline__ void stats_flush(double s[4], double *__restrict__ ou
 
 // Moments of turns *base + 1 .. *base + gridDim.x from the workgroup rows:
 // moments[t] = (n, mean_dt, sigma_dt, mean_dE, sigma_dE), sigma with ddof 0.
-__global__ void moments_reduce_kernel(const double *__restrict__ part, int grid, const int *base,
-                                      double n, double shift_t, double shift_e,
-                                      double *__restrict__ moments) {
-    __shared__ double s[4];
+// A workgroup a turn; the rows are added in index order.  They are brought to
+// LDS by all threads first: adding them as they are loaded is one trip to
+// memory after the other (196 rows a turn, 50 turns: 33 -> 5.6 us).
+constexpr int kMomentRows = 512;
+__global__ void __launch_bounds__(256) moments_reduce_kernel(const double *__restrict__ part,
+                                                             int grid, const int *base, double n,
+                                                             double shift_t, double shift_e,
+                                                             double *__restrict__ moments) {
+    __shared__ double s[4], rows[4 * kMomentRows];
     const int t = *base + 1 + blockIdx.x;
-    if (threadIdx.x < 4) {
-        double v = 0.0;
-        for (int g = 0; g < grid; ++g) v += part[((size_t)t * grid + g) * 4 + threadIdx.x];
-        s[threadIdx.x] = v;
+    double v = 0.0;
+    for (int g0 = 0; g0 < grid; g0 += kMomentRows) {
+        const int m = min(kMomentRows, grid - g0);
+        const double *src = part + ((size_t)t * grid + g0) * 4;
+        for (int j = threadIdx.x; j < 4 * m; j += blockDim.x) rows[j] = src[j];
+        __syncthreads();
+        if (threadIdx.x < 4) {
+#pragma unroll 8
+            for (int g = 0; g < m; ++g) v += rows[4 * g + threadIdx.x];
+        }
+        __syncthreads();
     }
+    if (threadIdx.x < 4) s[threadIdx.x] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         const double mt = s[0] / n, me = s[2] / n;
@@ -2170,7 +2183,7 @@ int Engine::finish_chunk(hipStream_t s, int count) {
                                (const double *)volt, volt32, n_slices);
     }
     if (stats_on) {
-        hipLaunchKernelGGL(moments_reduce_kernel, dim3(count), dim3(64), 0, s, d_stats, stats_grid,
+        hipLaunchKernelGGL(moments_reduce_kernel, dim3(count), dim3(256), 0, s, d_stats, stats_grid,
                            d_base, (double)n, stat_shift_t, stat_shift_e, d_moments);
         int rc = blmi_check_launch("moments_reduce");
         if (rc) return rc;

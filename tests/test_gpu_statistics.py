@@ -43,6 +43,34 @@ def test_fused_moments_match_numpy_of_oracle_turns(n_particles):
     np.testing.assert_array_equal(host(w.beam.dt), st["dt"])
 
 
+@pytest.mark.parametrize("n_particles,blocks_per_cu,block", [
+    (2, 1, 1024),  # one workgroup's row
+    (2 * 256 * 7 + 1, 1, 256),  # a few
+    (2 * 256 * 512, 2, 256),  # a full batch of rows on 256 CUs
+    (2 * 256 * 513 + 1, 3, 256),  # one row more
+    (600_001, 4, 256),  # two batches
+])
+def test_moments_at_row_counts(n_particles, blocks_per_cu, block):
+    """The sum over the workgroups' rows at the edges of its batches, to the
+    bars of the test above (n = 2: the spread by the same rule)."""
+    from blond_amd.trackers.fused import FusedTracker
+
+    w = build_workload("c1", n_particles=n_particles, n_turns=6, n_slices=100)
+    st = w.snapshot()
+    ft = FusedTracker(w.tracker, w.profile, None, statistics=True, block=block,
+                      blocks_per_cu=blocks_per_cu)
+    ft.track(4)
+    rows = ft.statistics(1, 4)
+    for t in range(4):
+        st = orc.track(st, 1, ORC)
+        dt, dE = st["dt"], st["dE"]
+        assert rows[t, 0] == n_particles
+        assert abs(rows[t, 1] - dt.mean()) <= 1e-12 * dt.std()
+        assert abs(rows[t, 3] - dE.mean()) <= 1e-12 * dE.std()
+        assert rows[t, 2] == pytest.approx(dt.std(), rel=1e-10)
+        assert rows[t, 4] == pytest.approx(dE.std(), rel=1e-10)
+
+
 def test_statistics_do_not_change_the_turns():
     a = build_workload("c2", n_particles=200001, n_turns=30, n_slices=1024, n_fft=4096)
     b = build_workload("c2", n_particles=200001, n_turns=30, n_slices=1024, n_fft=4096)
