@@ -37,7 +37,7 @@ struct Adjoint {
     double *d_x0 = nullptr;    // [2][np]: dt, dE at turn 0
     double *d_work = nullptr;  // [2][np]
     double *d_ckpt = nullptr;  // [n_ckpt][2][np] (entry 0 unused: d_x0 holds turn 0)
-    double *d_slots = nullptr; // [every][2][np]
+    double *d_slots = nullptr; // [every][np]: dt
     double *d_lam = nullptr;   // [2][np]: adjoints of dt, dE
     // slice axis
     unsigned long long *d_dep = nullptr;  // [kAdjRing][copies][n_slices] fixed-point deposit

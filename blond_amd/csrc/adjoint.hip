@@ -47,9 +47,9 @@
 // corr[m] = sum_t sum_i lV_t[i] p_t[(i - m) mod n_fft], from which the host
 // forms dL/dZ-parameters as -scale * sum_m irfft(dZ/dtheta)[m] corr[m].
 //
-// Traffic per macroparticle-turn: 32 B forward, 16 B recompute (the states of
-// a segment are written; the particles stay in registers), 48 B reverse
-// (state read, two adjoints read and written).
+// Traffic per macroparticle-turn: 32 B forward, 8 B recompute (the dt of a
+// segment's states are written; the particles stay in registers), 48 B reverse
+// (dt_t and dt_{t+1} read, two adjoints read and written).
 //
 // One launch a turn in each direction up to kAdjFuseSlices slices: every
 // particle workgroup forms the turn's slice-axis product (V_t from p_t, or
@@ -490,20 +490,21 @@ __global__ void __launch_bounds__(kAdjBlock) adj_turn_kernel(const double *xi, c
 }
 
 // ---------------------------------------------------------------------------
-// States t0 + 1 .. t1 - 1 of a segment from state t0, into slots 0, 1, ...
-// (stride pn doubles).  The segment's voltages are known, so nothing joins
-// the particles between its turns: they stay in registers, two pairs a
-// thread, and each turn only writes its state (16 B a macroparticle, where a
-// launch a turn reads and writes 32: 3.9 us a turn at 1e6 against 8.6 and a
-// launch gap).  A turn's table is built in one of two
-// LDS buffers while the turn before uses the other; its voltages are loaded
-// a turn ahead.
+// dt of states t0 + 1 .. t1 - 1 of a segment from state t0, into slots 0, 1, ...
+// (stride np doubles): the map is linear in dE, so the reverse pass needs no
+// more.  The segment's voltages are known, so nothing joins the particles
+// between its turns: they stay in registers, two pairs a thread, and each turn
+// only writes (8 B a macroparticle, where a launch a turn reads and writes 32:
+// 3.2 us a turn at 1e6, 2.5 of them arithmetic, against 8.6 and a launch gap;
+// 3.8 with dE written too).  A turn's table is built in one of two LDS buffers
+// while the turn before uses the other; its voltages are loaded a turn ahead
+// (its RF programs too: measured the same).
 // ---------------------------------------------------------------------------
 static size_t adj_segment_lds(int ns) { return sizeof(double) * 6 * (size_t)ns; }
 
 template <int MAP>
 __global__ void __launch_bounds__(kAdjBlock) adj_segment_kernel(const double *xi, const double *ei,
-                                                                double *slots, size_t pn,
+                                                                double *slots, int64_t np,
                                                                 int64_t n, int t0, int t1,
                                                                 AdjArgs a) {
     extern __shared__ __align__(16) double sh_seg[];
@@ -515,7 +516,7 @@ __global__ void __launch_bounds__(kAdjBlock) adj_segment_kernel(const double *xi
     cephes_tab_fill((LdsDoublePtr)sin_tab);
     const LdsConstDoublePtr stab = (LdsConstDoublePtr)sin_tab;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    const int64_t n2 = (n + 1) / 2, np = (int64_t)(pn / 2);
+    const int64_t n2 = (n + 1) / 2;
     // kAdjMaxSlices <= kAdjBlock: one slice a thread
     const int b = threadIdx.x;
     const bool has = MAP == kMapReference ? b < ns - 1 : b < ns;
@@ -553,19 +554,13 @@ __global__ void __launch_bounds__(kAdjBlock) adj_segment_kernel(const double *xi
             const TurnConst c(a, t);
             const double2 *tb = tab[t & 1];
             const double *vb = vl[t & 1];
-            double *xo = slots + (size_t)(t - t0) * pn, *eo = xo + np;
+            double *xo = slots + (size_t)(t - t0) * np;
             forward_step<MAP>(x0.x, e0.x, tb, vb, c, stab, a);
             forward_step<MAP>(x0.y, e0.y, tb, vb, c, stab, a);
             forward_step<MAP>(x1.x, e1.x, tb, vb, c, stab, a);
             forward_step<MAP>(x1.y, e1.y, tb, vb, c, stab, a);
-            if (hi) {
-                reinterpret_cast<double2 *>(xo)[i] = x0;
-                reinterpret_cast<double2 *>(eo)[i] = e0;
-            }
-            if (hj) {
-                reinterpret_cast<double2 *>(xo)[j] = x1;
-                reinterpret_cast<double2 *>(eo)[j] = e1;
-            }
+            if (hi) reinterpret_cast<double2 *>(xo)[i] = x0;
+            if (hj) reinterpret_cast<double2 *>(xo)[j] = x1;
             if (t + 1 < t1 - 1) put(t + 1);
         }
     }
@@ -642,39 +637,41 @@ __global__ void __launch_bounds__(kAdjSliceBlock) adj_profile_kernel(AdjArgs a, 
 }
 
 // ---------------------------------------------------------------------------
-// Reverse turn t (state (x, e) at turn t): see the file comment.  FUSE:
+// Reverse turn t (xs, x1s: dt_t and dt_{t+1}): see the file comment.  FUSE:
 // lp_{t+1} is formed here from lV_{t+1}; else it is read from a.lp.  Pairs of
 // macroparticles as in adj_turn_kernel (the pad slot's adjoints stay zero),
 // one pair ahead (two take 18.9 us in place of 17.2: 1e6 macroparticles).
-// LDS: lp_{t+1}, lV_t, the table (reference map) or V_t, the bin centres, and
-// with FUSE the product's words.
+// dt_{t+1} is read, not formed again from dE_t: the same traffic, one step of
+// the map less (16.5 -> 15.6 us at 1e6 macroparticles), and half the slots.
+// LDS: lp_{t+1}, lV_t, the kick's slopes (reference map) or V_t, the bin
+// centres, and with FUSE the product's words.
 // ---------------------------------------------------------------------------
 static size_t adj_reverse_lds(int ns, bool fuse) {
-    return sizeof(double) * (5 * (size_t)ns + (fuse ? prod_words(ns) : 0));
+    return sizeof(double) * (4 * (size_t)ns + (fuse ? prod_words(ns) : 0));
 }
 
 template <int MAP, bool FUSE>
 __global__ void __launch_bounds__(kAdjBlock) adj_reverse_kernel(const double *__restrict__ xs,
-                                                                const double *__restrict__ es,
+                                                                const double *__restrict__ x1s,
                                                                 double *__restrict__ lam_x,
                                                                 double *__restrict__ lam_e,
                                                                 int64_t n, int t, int last,
                                                                 AdjArgs a) {
     extern __shared__ __align__(16) double shr[];
-    double2 *tab = reinterpret_cast<double2 *>(shr);
-    double *vl = shr;  // spline map: V_t in the table's place
-    double *lp = shr + 2 * a.ns, *lvs = shr + 3 * a.ns, *bcs = shr + 4 * a.ns;
+    double *slope = shr;
+    double *vl = shr;  // spline map: V_t in the slopes' place
+    double *lp = shr + a.ns, *lvs = shr + 2 * a.ns, *bcs = shr + 3 * a.ns;
     __shared__ double red[kAdjWaves][2 * kAdjMaxRf];
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     const int64_t i_first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t n2 = (n + 1) / 2;
     struct Pair {
-        double2 x{}, e{}, lx{}, le{};
+        double2 x{}, x1{}, lx{}, le{};
     };
     auto load = [&](int64_t i, Pair &p) {
         if (i >= n2) return;
         p.x = reinterpret_cast<const double2 *>(xs)[i];
-        p.e = reinterpret_cast<const double2 *>(es)[i];
+        p.x1 = reinterpret_cast<const double2 *>(x1s)[i];
         p.lx = reinterpret_cast<const double2 *>(lam_x)[i];
         p.le = reinterpret_cast<const double2 *>(lam_e)[i];
     };
@@ -693,13 +690,13 @@ __global__ void __launch_bounds__(kAdjBlock) adj_reverse_kernel(const double *__
         if (product) l = ring_sum(a.lv, t + 1, ns, b);
         if (MAP == kMapReference) {
             bcs[b] = bcb;
-            if (b < ns - 1) tab[b] = interp_pair(v0, v1, bcb, a);
+            if (b < ns - 1) slope[b] = interp_pair(v0, v1, bcb, a).x;
         } else {
             vl[b] = v0;
         }
     }
     if (product) {
-        double *prod = shr + 5 * ns;
+        double *prod = shr + 4 * ns;
         g = prod_load_g<-1>(a);
         if (blockIdx.x == 0 && b < ns) a.lvh[(size_t)(t + 1) * ns + b] = l;
         prod_put(prod, g, l, a);
@@ -713,33 +710,28 @@ __global__ void __launch_bounds__(kAdjBlock) adj_reverse_kernel(const double *__
     double gsum[2 * kAdjMaxRf];
 #pragma unroll
     for (int j = 0; j < 2 * kAdjMaxRf; ++j) gsum[j] = 0.0;
-    auto step = [&](double x, double e, double &lam_x_i, double &lam_e_i, bool own) {
-        // forward step t, as adj_turn_kernel
+    auto step = [&](double x, double x1, double &lam_x_i, double &lam_e_i, bool own) {
+        // the kicks of turn t and their derivatives
         double wk[3], dkick;
         int k;
-        double e1;
         if (MAP == kMapReference) {
             k = interp_bin(x, a);
-            const double2 se = tab[k >= 0 ? k : 0];
-            e1 = k >= 0 ? e + (x * se.x + se.y) : e;
-            dkick = k >= 0 ? se.x : 0.0;
+            const double sl = slope[k >= 0 ? k : 0];
+            dkick = k >= 0 ? sl : 0.0;
         } else {
-            e1 = e + induced_kick(vl, x, a, &dkick, wk, k);
+            induced_kick(vl, x, a, &dkick, wk, k);
         }
         // constant trip counts with a guard keep sn, cs and gsum in registers
         double sn[kAdjMaxRf], cs[kAdjMaxRf];
-        double s = 0.0, ds = 0.0;
+        double ds = 0.0;
 #pragma unroll
         for (int j = 0; j < kAdjMaxRf; ++j) {
             sn[j] = cs[j] = 0.0;
             if (j < a.n_rf) {
                 cephes_sincos(c.w[j] * x + c.phi[j], sn[j], cs[j]);
-                s = s + c.V[j] * sn[j];
                 ds = ds + c.V[j] * c.w[j] * cs[j];
             }
         }
-        const double e2 = e1 + (a.charge * s + c.acc);
-        const double x1 = x + c.coeff * e2;
         // deposit adjoint of p_{t+1} at x1
         double lx = lam_x_i;
         if (MAP == kMapReference) {
@@ -793,8 +785,8 @@ __global__ void __launch_bounds__(kAdjBlock) adj_reverse_kernel(const double *__
     for (int64_t i = i_first; i < n2; i += stride) {
         Pair p = next;
         load(i + stride, next);
-        step(p.x.x, p.e.x, p.lx.x, p.le.x, true);
-        step(p.x.y, p.e.y, p.lx.y, p.le.y, 2 * i + 1 < n);
+        step(p.x.x, p.x1.x, p.lx.x, p.le.x, true);
+        step(p.x.y, p.x1.y, p.lx.y, p.le.y, 2 * i + 1 < n);
         reinterpret_cast<double2 *>(lam_x)[i] = p.lx;
         reinterpret_cast<double2 *>(lam_e)[i] = p.le;
     }
@@ -955,7 +947,7 @@ int Adjoint::init(int64_t n_, int n_rf_, int n_turns_, int n_slices_, int every_
     BLMI_HIP_TRY(hipMemset(d_x0, 0, sizeof(double) * pn));  // the pad slots
     BLMI_HIP_TRY(hipMalloc(&d_work, sizeof(double) * pn));
     BLMI_HIP_TRY(hipMalloc(&d_ckpt, sizeof(double) * pn * n_ckpt));
-    BLMI_HIP_TRY(hipMalloc(&d_slots, sizeof(double) * pn * every));
+    BLMI_HIP_TRY(hipMalloc(&d_slots, sizeof(double) * (size_t)np * every));
     BLMI_HIP_TRY(hipMalloc(&d_lam, sizeof(double) * pn));
     BLMI_HIP_TRY(hipMalloc(&d_dep, sizeof(unsigned long long) * kAdjRing * kAdjCopies * n_slices));
     BLMI_HIP_TRY(hipMalloc(&d_prof, sizeof(double) * nt * n_slices));
@@ -1151,15 +1143,17 @@ static int enqueue_backward_map(Adjoint &j, int T, hipStream_t s) {
     if (rc) return rc;
     for (int seg = (T - 1) / every; seg >= 0; --seg) {
         const int t0 = seg * every, t1 = (t0 + every < T) ? t0 + every : T;
-        // state t0 is kept; t0 + 1 .. t1 - 1 go to slots 0 .. t1 - t0 - 2
+        // states t0 and t1 are kept; dt of t0 + 1 .. t1 - 1 go to slots 0 .. t1 - t0 - 2
         const double *s0 = state_at(j, t0, T);
+        const double *x1 = state_at(j, t1, T);
         if (t1 - t0 > 1)
             hipLaunchKernelGGL(adj_segment_kernel<MAP>, dim3(grid), dim3(kAdjBlock), lds_seg, s, s0,
-                               s0 + np, j.d_slots, pn, n, t0, t1, a);
+                               s0 + np, j.d_slots, np, n, t0, t1, a);
         for (int t = t1 - 1; t >= t0; --t) {
-            const double *st = t == t0 ? s0 : j.d_slots + (size_t)(t - t0 - 1) * pn;
+            const double *x0 = t == t0 ? s0 : j.d_slots + (size_t)(t - t0 - 1) * np;
             hipLaunchKernelGGL((adj_reverse_kernel<MAP, FUSE>), dim3(grid), dim3(kAdjBlock), lds_rev,
-                               s, st, st + np, j.d_lam, j.d_lam + np, n, t, T, a);
+                               s, x0, x1, j.d_lam, j.d_lam + np, n, t, T, a);
+            x1 = x0;
             if (!FUSE || t == 0)
                 hipLaunchKernelGGL(adj_iv_kernel, dim3(sgrid), dim3(kAdjSliceBlock), lds_slice, s, a,
                                    t, !FUSE && t > 0);
