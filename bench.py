@@ -412,7 +412,7 @@ def _adjoint(torch, turns, every, case=None, map="reference") -> dict:
     step()
     el = _timed(step, torch.cuda.synchronize)
     n = c.beam.n_macroparticles
-    bpp = 80 if every == 1 else 112  # forward 32 + reverse 48 (+ recompute 32)
+    bpp = 80 if every == 1 else 88  # forward 32 + reverse 48 (+ recompute 8)
     dtr.close()
     how = ("every turn's state kept in HBM, no recompute" if every == 1 else
            f"checkpoints every {every} turns with recomputation")

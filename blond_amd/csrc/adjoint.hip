@@ -268,8 +268,8 @@ __device__ __forceinline__ int prod_x_at(int j) { return 17 * ((j >> 4) + 15) + 
 // Largest slice count a prologue forms the product for (one G word and one
 // slice a thread, at most two tiles); above it the slice axis has launches of
 // its own.  1e6 macroparticles, 256 slices: forward 12.9 us a turn against 10.3
-// and 5.2 for the particle and the slice launch, reverse 17.3 against 13.7 and
-// 5.8, and a launch gap of about 1.4 us less in each; of the prologue about 2 us
+// and 5.2 for the particle and the slice launch, reverse 17.3 (15.6 since it
+// reads dt_{t+1}) against 13.7 and 5.8, and a launch gap of about 1.4 us less in each; of the prologue about 2 us
 // are the product.  It grows with the square of the slices on every CU: four
 // times the matrix work at 512, and at 1024 more (8 us) than the slice launch.
 constexpr int kAdjFuseSlices = 512;
