@@ -354,19 +354,48 @@ __global__ void irfft_lds_kernel(const double2 *__restrict__ in, int64_t m_in, d
 // ---------------------------------------------------------------------------
 // one-turn induced voltage on one workgroup
 // ---------------------------------------------------------------------------
+// FL > 0 launches take 512 threads (lds_threads of M <= 1024): the bound
+// leaves their registers room (no scratch spills)
+constexpr int kLdsWaveThreads = 512;
+
 // The profile is read from a.src, or as the sum of a.groups copies of u32
 // counts at cin (then cleared at cclr, which may equal cin: each element is
 // read before it is cleared, by the same thread).  FL: M as a constant when
-// it is a power of two in [16, 1024] (one wavefront a transform, twiddles
-// staged in LDS after the data), else 0 (workgroup-wide stages).
+// it is a power of two in [16, 1024] (one wavefront a transform), else 0
+// (workgroup-wide stages).  stage: the twiddles are staged in LDS after the
+// data (always with FL > 0).  One workgroup is bound by the latency of its
+// chain: what later steps read from memory is asked for before the profile
+// (256 bunches at once, 512 complex points: 15.0 -> 13.9 us; 1000 slices alone,
+// its twiddles now staged: 14.7 -> 12.3 us; the operands of the
+// spectrum's pairs held too there spill: 13.5 us).
 template <int FL>
 __device__ void induced_lds_body(const InducedArgs &a, const unsigned *cin, unsigned *cclr, int M,
                                  const StageList &st, const double2 *__restrict__ tw,
-                                 const double2 *__restrict__ tw2) {
+                                 const double2 *__restrict__ tw2, bool stage) {
     extern __shared__ double2 buf[];
     double2 *twl = buf + M;
-    if constexpr (FL > 0)
-        for (int j = threadIdx.x; j < M; j += blockDim.x) twl[j] = tw[j];
+    const int T = FL > 0 ? kLdsWaveThreads : (int)blockDim.x;
+    // pairs (k, M - k) of a thread: host guarantees M/2+1 <= PMAX * T
+    constexpr int PMAX = FL > 0 ? FL / 2 / kLdsWaveThreads + 1 : 8;
+    constexpr int PRE = FL > 0 ? PMAX : 0;  // pairs whose operands are loaded here
+    double2 wk[PMAX], wmk[PMAX], zk[PMAX], zmk[PMAX];
+#pragma unroll
+    for (int q = 0; q < PRE; ++q) {
+        const int k = threadIdx.x + q * T;
+        if (k <= M / 2) {
+            wk[q] = tw2[k];
+            wmk[q] = tw2[M - k];
+            zk[q] = a.Z[k];
+            zmk[q] = a.Z[M - k];
+        }
+    }
+    double inv_bw = 0.0, bc_pre = 0.0;
+    if (a.tab) {
+        inv_bw = interp_inv_bw(a.bc, a.n_slices, a.f32);
+        if ((int)threadIdx.x < a.n_slices - 1) bc_pre = a.bc[threadIdx.x];
+    }
+    if (FL > 0 || stage)
+        for (int j = threadIdx.x; j < M; j += T) twl[j] = tw[j];
     const int ns = a.n_slices;
     // load the profile as z[m] = p[2m] + i p[2m+1], zero padded to n = 2M
     auto prof = [&](int j) -> double {
@@ -395,33 +424,37 @@ __device__ void induced_lds_body(const InducedArgs &a, const unsigned *cin, unsi
     __syncthreads();
     if constexpr (FL > 0)
         wave_fft_batch<FL, false>(buf, 1, M, twl, (int)blockDim.x);
+    else if (stage)
+        fft_lds<false>(buf, M, st, twl);
     else
         fft_lds<false>(buf, M, st, tw);
     // spectrum -> times impedance -> half-length inverse input, pairwise.
     // All pairs are read into registers before any is overwritten.
-    constexpr int PMAX = 8;  // host guarantees M/2+1 <= PMAX * blockDim.x
     double2 ua[PMAX], ub[PMAX];
 #pragma unroll
     for (int q = 0; q < PMAX; ++q) {
-        const int k = threadIdx.x + q * blockDim.x;
+        const int k = threadIdx.x + q * T;
         if (k <= M / 2) {
+            const bool pre = q < PRE;
+            const double2 Wk = pre ? wk[q] : tw2[k], Wmk = pre ? wmk[q] : tw2[M - k];
             const double2 Zk = buf[k % M], Zmk = buf[(M - k) % M];
             double2 Xk, Xmk;
-            real_split(Zk, Zmk, tw2[k], tw2[M - k], Xk, Xmk);
+            real_split(Zk, Zmk, Wk, Wmk, Xk, Xmk);
             // impedance.py:479-484: total_impedance * beam_spectrum
-            double2 Yk = cmul(a.Z[k], Xk), Ymk = cmul(a.Z[M - k], Xmk);
+            double2 Yk = cmul(pre ? zk[q] : a.Z[k], Xk);
+            double2 Ymk = cmul(pre ? zmk[q] : a.Z[M - k], Xmk);
             if (k == 0) {  // c2r ignores the imaginary parts of DC and Nyquist
                 Yk.y = 0.0;
                 Ymk.y = 0.0;
             }
-            ua[q] = real_merge(Yk, Ymk, tw2[k]);
-            ub[q] = real_merge(Ymk, Yk, tw2[M - k]);
+            ua[q] = real_merge(Yk, Ymk, Wk);
+            ub[q] = real_merge(Ymk, Yk, Wmk);
         }
     }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < PMAX; ++q) {
-        const int k = threadIdx.x + q * blockDim.x;
+        const int k = threadIdx.x + q * T;
         if (k <= M / 2) {
             buf[k % M] = ua[q];
             if (k != 0 && 2 * k != M) buf[M - k] = ub[q];
@@ -430,6 +463,8 @@ __device__ void induced_lds_body(const InducedArgs &a, const unsigned *cin, unsi
     __syncthreads();
     if constexpr (FL > 0)
         wave_fft_batch<FL, true>(buf, 1, M, twl, (int)blockDim.x);
+    else if (stage)
+        fft_lds<true>(buf, M, st, twl);
     else
         fft_lds<true>(buf, M, st, tw);
     // V = -(charge*e*ratio * irfft(...))[:n_slices]   (impedance.py:475-489)
@@ -448,26 +483,22 @@ __device__ void induced_lds_body(const InducedArgs &a, const unsigned *cin, unsi
     if (a.tab) {
         __syncthreads();
         // linear_interp_kick.cpp:33-48 on V (acc = 0 for the induced kick)
-        const double inv_bw = interp_inv_bw(a.bc, ns, a.f32);
         if (threadIdx.x == 0) {
             a.tab_params[0] = a.bc[0];
             a.tab_params[1] = inv_bw;
         }
-        for (int i = threadIdx.x; i < ns - 1; i += blockDim.x)
-            store_interp_entry(a.tab, i,
-                               interp_entry(vl[i], vl[i + 1], a.bc[i], a.charge, inv_bw, a.f32),
+        for (int i = threadIdx.x; i < ns - 1; i += T) {
+            const double b = i < T ? bc_pre : a.bc[i];
+            store_interp_entry(a.tab, i, interp_entry(vl[i], vl[i + 1], b, a.charge, inv_bw, a.f32),
                                a.f32);
+        }
     }
 }
 
-// FL > 0 launches take 512 threads (lds_threads of M <= 1024): the bound
-// leaves their registers room (no scratch spills)
-constexpr int kLdsWaveThreads = 512;
-
 template <int FL>
 __global__ void __launch_bounds__(FL > 0 ? kLdsWaveThreads : 1024)
-    induced_lds_kernel(InducedArgs a, int M, StageList st,
-                                   const double2 *__restrict__ tw, const double2 *__restrict__ tw2) {
+    induced_lds_kernel(InducedArgs a, int M, StageList st, const double2 *__restrict__ tw,
+                       const double2 *__restrict__ tw2, bool stage) {
     const unsigned *cin = nullptr;
     unsigned *cclr = nullptr;
     if (a.counts0) {
@@ -475,7 +506,7 @@ __global__ void __launch_bounds__(FL > 0 ? kLdsWaveThreads : 1024)
         cin = (t & 1) ? a.counts1 : a.counts0;
         cclr = (t & 1) ? a.counts0 : a.counts1;
     }
-    induced_lds_body<FL>(a, cin, cclr, M, st, tw, tw2);
+    induced_lds_body<FL>(a, cin, cclr, M, st, tw, tw2, stage);
 }
 
 // One workgroup per bunch: bunch b's arguments are args[b]; its counts (one
@@ -484,9 +515,9 @@ template <int FL>
 __global__ void __launch_bounds__(FL > 0 ? kLdsWaveThreads : 1024)
     induced_lds_batch_kernel(const InducedArgs *__restrict__ args, int M, StageList st,
                                          const double2 *__restrict__ tw,
-                                         const double2 *__restrict__ tw2) {
+                                         const double2 *__restrict__ tw2, bool stage) {
     const InducedArgs a = args[blockIdx.x];
-    induced_lds_body<FL>(a, a.counts0, a.counts0, M, st, tw, tw2);
+    induced_lds_body<FL>(a, a.counts0, a.counts0, M, st, tw, tw2, stage);
 }
 
 // ---------------------------------------------------------------------------
@@ -1027,13 +1058,15 @@ struct LdsKernels {
     decltype(&induced_lds_kernel<0>) one = induced_lds_kernel<0>;
     decltype(&induced_lds_batch_kernel<0>) batch = induced_lds_batch_kernel<0>;
     size_t lds = 0;
+    bool stage = false;  // twiddles in LDS
 };
 
 static LdsKernels lds_kernels(int M, int threads) {
     LdsKernels k;
     const bool wave = wave_len(M) && threads == kLdsWaveThreads;
     if (wave) pick_lds_kernels<16>(M, k.one, k.batch);
-    k.lds = sizeof(double2) * (size_t)M * (wave ? 2 : 1);
+    k.stage = wave || 2 * sizeof(double2) * (size_t)M <= (size_t)device_max_lds();
+    k.lds = sizeof(double2) * (size_t)M * (k.stage ? 2 : 1);
     return k;
 }
 
@@ -1048,7 +1081,8 @@ int launch_induced_voltage_lds(const InducedArgs &a, const FftPlan &p, hipStream
     const LdsKernels k = lds_kernels(p.M, p.threads);
     int rc = set_lds_limit((const void *)k.one, k.lds);
     if (rc) return rc;
-    launch(k.one, dim3(1), dim3(p.threads), k.lds, s, ev, a, p.M, stages_of(p), p.tw, p.tw2);
+    launch(k.one, dim3(1), dim3(p.threads), k.lds, s, ev, a, p.M, stages_of(p), p.tw, p.tw2,
+           k.stage);
     return blmi_check_launch("induced_voltage");
 }
 
@@ -1064,7 +1098,7 @@ int launch_induced_lds_batch(const InducedArgs *d_args, int n_bunches, int n_sli
     int rc = set_lds_limit((const void *)k.batch, k.lds);
     if (rc) return rc;
     launch(k.batch, dim3(n_bunches), dim3(p.threads), k.lds, s, ev, d_args, p.M, stages_of(p), p.tw,
-           p.tw2);
+           p.tw2, k.stage);
     return blmi_check_launch("induced_voltage_batch");
 }
 

@@ -37,6 +37,17 @@ def test_direct_convolution_shapes(n_slices, groups):
     _first_turn(w, groups=groups, method="direct")
 
 
+# one workgroup's transform: one wavefront a transform at both ends of its
+# range and with two pairs a thread, workgroup-wide stages with their twiddles
+# in LDS up to where both fit 160 KiB (n_fft 10240) and from memory above
+@pytest.mark.parametrize("n_slices,n_fft", [
+    (3, 6), (16, 32), (15, 30), (500, 1000), (1024, 1024), (1025, 2048), (1000, 2160),
+    (2000, 8192), (2048, 10240), (2048, 10800)])
+def test_one_workgroup_transform(n_slices, n_fft):
+    _first_turn(build_workload("c2", n_particles=20001, n_turns=3, n_slices=n_slices, n_fft=n_fft),
+                method="fft")
+
+
 # pairs a thread 1 and 2 of 256, 512 and 1024 threads a workgroup on 256 CUs,
 # and one macroparticle to either side
 @pytest.mark.parametrize("pairs", [1, 65536, 131072, 262144, 3 * 262144])
