@@ -96,11 +96,25 @@ __device__ inline void feedback_turn_body(const FeedbackArgs &a, int part = 0) {
         wdj = a.omega_d[(size_t)(t + 1) * nr + j];
         dpj = dphi_rf[j];
     }
+    // thread 0's: the programs of the turn and the loop's state (no part
+    // writes it before every part has read it and arrived).  Read with the end
+    // points' terms as the control law ran, they were most of the serial tail
+    // (1024 slices, with the convolution: 7.7 -> 7.1 us)
+    double prv[kFbCols], st[kFbState], wd = 0.0;
+    if (active && threadIdx.x == 0) {
+        const double *pr = a.prog + (size_t)t * kFbCols;
+#pragma unroll
+        for (int k = 0; k < kFbCols; ++k) prv[k] = pr[k];
+#pragma unroll
+        for (int k = 0; k < kFbState; ++k) st[k] = a.state[k];
+        wd = a.omega_d[(size_t)t * nr];
+    }
     double on_time_pc = 0.0;  // PSB: the loop turn the counter points at
     if (active && a.machine == kFbPSB && threadIdx.x == 0) {
-        const int pc = (int)a.state[kFbPLCounter];
+        const int pc = (int)st[kFbPLCounter];
         if (pc < a.n_on_time) on_time_pc = a.on_time[pc];
     }
+    __shared__ double ends_sh[4];
     if (active) {
         const unsigned *cin = nullptr;
         if (a.from_counts || (a.pending && a.pending[t & 1] == t))
@@ -124,6 +138,12 @@ __device__ inline void feedback_turn_body(const FeedbackArgs &a, int part = 0) {
         } else {
             // trapz_const_delta split by interior index over the parts
             const int n = ns - b0;
+            // the end points of every part: two lanes of its last wavefront,
+            // beside the interior, so that the last part to arrive has them
+            if ((int)threadIdx.x >= (int)blockDim.x - 2) {
+                const int e = (int)blockDim.x - 1 - (int)threadIdx.x;
+                f(e ? n - 1 : 0, ends_sh[2 * e], ends_sh[2 * e + 1]);
+            }
             double ps = 0.0, pc = 0.0;
             for (int i = 1 + part * (int)blockDim.x + (int)threadIdx.x; i < n - 1;
                  i += n_parts * (int)blockDim.x) {
@@ -153,30 +173,24 @@ __device__ inline void feedback_turn_body(const FeedbackArgs &a, int part = 0) {
                                             __HIP_MEMORY_SCOPE_AGENT);
                 }
                 __hip_atomic_store(a.arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                double s0, c0, s1, c1;
-                f(0, s0, c0);
-                f(n - 1, s1, c1);
-                const double psum_s = (s0 + s1) / 2. + ss;
-                const double psum_c = (c0 + c1) / 2. + sc;
+                const double psum_s = (ends_sh[0] + ends_sh[2]) / 2. + ss;
+                const double psum_c = (ends_sh[1] + ends_sh[3]) / 2. + sc;
                 coeff = (a.bin_size * psum_s) / (a.bin_size * psum_c);
             }
         }
         if (threadIdx.x == 0) {
-            const double *pr = a.prog + (size_t)t * kFbCols;
-            double *st = a.state;
             // beam_feedback.py:282-286, 317-322
             const double phi_beam = atan(coeff) + M_PI;
-            const double dphi = phi_beam - pr[kFbPhiS];
-            const double wd = a.omega_d[(size_t)t * nr];
+            const double dphi = phi_beam - prv[kFbPhiS];
             double domega = 0.0;
             if (a.machine == kFbLHC) {
                 // beam_feedback.py:545-561
-                const double x = dphi_rf[0] + a.reference;
-                domega = -pr[kFbGain] * dphi - pr[kFbGain2P] * (st[kFbLhcY] + pr[kFbLhcA] * x);
-                st[kFbLhcY] = (1 - pr[kFbLhcT]) * st[kFbLhcY] + (1 - pr[kFbLhcA]) * pr[kFbLhcT] * x;
+                const double x = dpj + a.reference;  // thread 0: dphi_rf[0]
+                domega = -prv[kFbGain] * dphi - prv[kFbGain2P] * (st[kFbLhcY] + prv[kFbLhcA] * x);
+                st[kFbLhcY] = (1 - prv[kFbLhcT]) * st[kFbLhcY] + (1 - prv[kFbLhcA]) * prv[kFbLhcT] * x;
             } else if (a.machine == kFbLHC_F) {
                 // beam_feedback.py:414-441
-                domega = -pr[kFbGain] * dphi - pr[kFbGain2P] * (omega - wd + a.reference);
+                domega = -prv[kFbGain] * dphi - prv[kFbGain2P] * (omega - wd + a.reference);
             } else {
                 // beam_feedback.py:563-622
                 st[kFbDphiSum] += dphi;
@@ -185,15 +199,15 @@ __device__ inline void feedback_turn_body(const FeedbackArgs &a, int part = 0) {
                     const int prev = pc - 1 < 0 ? a.n_on_time - 1 : pc - 1;
                     st[kFbDphiAv] = st[kFbDphiSum] / (a.on_time[pc] - a.on_time[prev]);
                     st[kFbDomegaPL] = 0.99803799 * st[kFbDomegaPL] +
-                                      pr[kFbGain] * (0.99901903 * st[kFbDphiAv] -
+                                      prv[kFbGain] * (0.99901903 * st[kFbDphiAv] -
                                                      0.99901003 * st[kFbDphiAvPrev]);
                     st[kFbDphiAvPrev] = st[kFbDphiAv];
                     st[kFbDphiSum] = 0.0;
-                    const double g = pr[kFbGamma];
-                    st[kFbDROverR] = (omega - wd) / (wd * (1.0 / (pr[kFbAlpha0] * (g * g)) - 1.0));
+                    const double g = prv[kFbGamma];
+                    st[kFbDROverR] = (omega - wd) / (wd * (1.0 / (prv[kFbAlpha0] * (g * g)) - 1.0));
                     st[kFbDomegaRL] = st[kFbDomegaRL] +
-                                      pr[kFbGain2P] * (st[kFbDROverR] - st[kFbDROverRPrev]) +
-                                      pr[kFbGain2I] * st[kFbDROverR];
+                                      prv[kFbGain2P] * (st[kFbDROverR] - st[kFbDROverRPrev]) +
+                                      prv[kFbGain2I] * st[kFbDROverR];
                     st[kFbDROverRPrev] = st[kFbDROverR];
                     st[kFbPLCounter] = (double)(pc + 1);
                 }
@@ -202,6 +216,8 @@ __device__ inline void feedback_turn_body(const FeedbackArgs &a, int part = 0) {
             st[kFbDomegaRf] = domega;
             st[kFbPhiBeam] = phi_beam;
             st[kFbDphi] = dphi;
+#pragma unroll
+            for (int k = 0; k < kFbState; ++k) a.state[k] = st[k];
             domega_sh = domega;
         }
     }

@@ -134,6 +134,18 @@ def test_feedback_turns_fused_with_intensity(kind, n_slices):
     _check(w, ref)
 
 
+@pytest.mark.parametrize("n_slices", (255, 256, 257, 258, 513, 1026))
+@pytest.mark.parametrize("kind", ("LHC", "PSB"))
+def test_loop_parts_at_slice_edges(kind, n_slices):
+    """The sums' end points and parts where one part becomes two and a part
+    has a single interior bin, over the first turns (bars as above)."""
+    w = build_feedback_workload(kind, n_particles=40001, n_turns=10, n_slices=n_slices,
+                                intensity=True)
+    ref = _ref(w, 4)
+    w.fused(4)
+    _check(w, ref)
+
+
 def test_feedback_fused_graph_vs_eager_and_object_by_object():
     a = build_feedback_workload("PSB", n_particles=30001, n_turns=80)
     b = build_feedback_workload("PSB", n_particles=30001, n_turns=80)
