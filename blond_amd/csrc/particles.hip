@@ -310,7 +310,7 @@ BLMI_INST(float)
 // Workgroups: one of 512 threads per CU at most.  Their rows are summed by
 // whoever needs them (every workgroup of the second pass, then the last
 // launch), one row a thread: read one after the other by a single thread, the
-// 4096 rows of 1e6 macroparticles took 427 us in each of two launches, and the
+// 3907 rows of 1e6 macroparticles took 427 us in each of two launches, and the
 // whole call's launches 876 us; now 17.7 us (5e4 macroparticles: 63 -> 14.6 us).
 // Two passes over 16 or 24 B a macroparticle, which the last-level cache
 // holds for the second up to about 1e7.

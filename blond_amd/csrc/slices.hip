@@ -26,15 +26,33 @@ __device__ __forceinline__ int hist_bin(T t, T cut_left, T inv_bw, int n_slices)
     return (f >= T(0) && f < T(n_slices)) ? (int)f : -1;
 }
 
-// One workgroup of 1024 threads per CU at most: at the end every workgroup
-// adds its bins to the output, and one address takes a device-scope atomic
-// about every 25 ns, so the flush costs 25 ns times the workgroups that hold
-// a bin.  1e6 macroparticles on 1000 slices: 24.1 us with 977 workgroups of
-// 256 threads, 8.0 us with 256 of 1024.  Four pairs a thread are loaded
-// before the first is counted (16 wavefronts a CU with one pair each leave
-// the memory system idle).
+// With the bins in LDS, one workgroup of 1024 threads per CU at most: at the
+// end every workgroup adds its bins to the output, and one address takes a
+// device-scope atomic about every 25 ns, so the flush costs 25 ns times the
+// workgroups that hold a bin.  1e6 macroparticles on 1000 slices: 28.4 us with
+// 1024 workgroups of 256 threads, 9.1 us with 256 of 1024.  A thread with four
+// pairs or more (n > 2.1e6) loads four before it counts the first: 3e6
+// macroparticles 36.3 -> 10.1 us, 1e7 36.0 -> 17.5 us.
+// With the bins in memory (kHistGlobalBlock) every macroparticle is a
+// device-scope atomic and the rate of those is the bound, about 20 a ns (less
+// where they meet in few bins); the shape matters for small bunches only,
+// which many small workgroups spread over the CUs (1e4 macroparticles, smooth,
+// 16384 slices: 11.0 us, and 13.6 in workgroups of 1024; 1e6: 98.8 in either).
 constexpr int kHistBlock = 1024;
+constexpr int kHistGlobalBlock = 256;
 constexpr int kHistUnroll = 4;
+
+struct HistShape {
+    int grid, block;
+};
+static HistShape hist_shape(int64_t items, bool lds) {
+    HistShape h;
+    h.block = lds ? kHistBlock : kHistGlobalBlock;
+    h.grid = stream_grid(items, h.block);
+    const int cap = device_cu_count() * (lds ? 1 : 4);
+    if (h.grid > cap) h.grid = cap;
+    return h;
+}
 
 template <typename T, int VEC, bool LDS>
 __global__ void __launch_bounds__(kHistBlock) histogram_kernel(const T *__restrict__ dt, int64_t n,
@@ -116,22 +134,21 @@ int launch_histogram(const T *dt, int64_t n, T *profile, T cut_left, T cut_right
     const size_t lds = (size_t)n_slices * sizeof(unsigned);
     const bool use_lds = lds <= 65536;
     const bool vec = aligned16(dt);
-    int grid = stream_grid(vec ? (n + 1) / 2 : n, kHistBlock);
-    if (use_lds && grid > device_cu_count()) grid = device_cu_count();
-    const dim3 block(kHistBlock);
+    const HistShape h = hist_shape(vec ? (n + 1) / 2 : n, use_lds);
+    const dim3 grid(h.grid), block(h.block);
     if (use_lds) {
         if (vec)
-            hipLaunchKernelGGL((histogram_kernel<T, 2, true>), dim3(grid), block, lds, s, dt, n,
+            hipLaunchKernelGGL((histogram_kernel<T, 2, true>), grid, block, lds, s, dt, n,
                                profile, cut_left, inv_bw, n_slices);
         else
-            hipLaunchKernelGGL((histogram_kernel<T, 1, true>), dim3(grid), block, lds, s, dt, n,
+            hipLaunchKernelGGL((histogram_kernel<T, 1, true>), grid, block, lds, s, dt, n,
                                profile, cut_left, inv_bw, n_slices);
     } else {
         if (vec)
-            hipLaunchKernelGGL((histogram_kernel<T, 2, false>), dim3(grid), block, 0, s, dt, n,
+            hipLaunchKernelGGL((histogram_kernel<T, 2, false>), grid, block, 0, s, dt, n,
                                profile, cut_left, inv_bw, n_slices);
         else
-            hipLaunchKernelGGL((histogram_kernel<T, 1, false>), dim3(grid), block, 0, s, dt, n,
+            hipLaunchKernelGGL((histogram_kernel<T, 1, false>), grid, block, 0, s, dt, n,
                                profile, cut_left, inv_bw, n_slices);
     }
     return blmi_check_launch("histogram");
@@ -194,16 +211,15 @@ int launch_sparse_histogram(const T *dt, int64_t n, T *profile, const T *cut_lef
     int rc = launch_fill<T>(profile, total, T(0), s);
     if (rc || n <= 0) return rc;
     const size_t lds = (size_t)total * sizeof(unsigned);
-    // one workgroup per CU with an LDS histogram, as histogram_kernel
-    int grid = stream_grid(n, kHistBlock);
-    if (lds <= 65536 && grid > device_cu_count()) grid = device_cu_count();
+    const HistShape h = hist_shape(n, lds <= 65536);
+    const dim3 grid(h.grid), block(h.block);
     if (lds <= 65536)
-        hipLaunchKernelGGL((sparse_hist_kernel<T, true>), dim3(grid), dim3(kHistBlock), lds, s, dt, n,
-                           profile, cut_left, cut_right, bunch_indexes, n_slices_bucket, n_filled,
+        hipLaunchKernelGGL((sparse_hist_kernel<T, true>), grid, block, lds, s, dt, n, profile,
+                           cut_left, cut_right, bunch_indexes, n_slices_bucket, n_filled,
                            n_pattern);
     else
-        hipLaunchKernelGGL((sparse_hist_kernel<T, false>), dim3(grid), dim3(kHistBlock), 0, s, dt, n,
-                           profile, cut_left, cut_right, bunch_indexes, n_slices_bucket, n_filled,
+        hipLaunchKernelGGL((sparse_hist_kernel<T, false>), grid, block, 0, s, dt, n, profile,
+                           cut_left, cut_right, bunch_indexes, n_slices_bucket, n_filled,
                            n_pattern);
     return blmi_check_launch("sparse_histogram");
 }
@@ -304,14 +320,13 @@ int launch_smooth_histogram(const T *dt, int64_t n, T *profile, T cut_left, T cu
     if (rc) return rc;
     if (n > 0) {
         const size_t lds = (size_t)n_slices * sizeof(unsigned long long);
-        // one workgroup per CU with LDS sums, as histogram_kernel
-        int grid = stream_grid(n, kHistBlock);
-        if (lds <= 65536 && grid > device_cu_count()) grid = device_cu_count();
+        const HistShape h = hist_shape(n, lds <= 65536);
+        const dim3 grid(h.grid), block(h.block);
         if (lds <= 65536)
-            hipLaunchKernelGGL((smooth_kernel<T, true>), dim3(grid), dim3(kHistBlock), lds, s, dt, n, acc,
+            hipLaunchKernelGGL((smooth_kernel<T, true>), grid, block, lds, s, dt, n, acc,
                                cut_left, inv_bw, lo, hi, n_slices, scale);
         else
-            hipLaunchKernelGGL((smooth_kernel<T, false>), dim3(grid), dim3(kHistBlock), 0, s, dt, n, acc,
+            hipLaunchKernelGGL((smooth_kernel<T, false>), grid, block, 0, s, dt, n, acc,
                                cut_left, inv_bw, lo, hi, n_slices, scale);
         rc = blmi_check_launch("smooth_histogram");
         if (rc) return rc;

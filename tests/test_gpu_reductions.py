@@ -52,6 +52,32 @@ def test_histograms_at_loop_edges(n, shift):
     assert np.max(np.abs(got.cpu().numpy() - ref)) <= max(tol, 1e-300)
 
 
+# more bins than LDS holds: one, a few and all of the small workgroups of the
+# path that counts in memory (256 threads, 1024 of them), and two rounds
+@pytest.mark.parametrize("n", [1, 255, 513, 20001, 262143, 2 * 262144 + 1, 1100003])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_histograms_with_the_bins_in_memory(n, shift):
+    import torch
+
+    from blond_amd.utils import bmath as bm
+
+    dt, _ = _bunch(n, n)
+    lib = orc.oracle_lib()
+    x = _device(dt, shift)
+    ref = np.zeros(16385)
+    lib.slice_beam(dt, ref, 0.0, 2.5e-9)
+    got = torch.full((16385,), 7.0, dtype=torch.float64, device="cuda")
+    bm.slice_beam(x, got, 0.0, 2.5e-9)
+    assert np.array_equal(got.cpu().numpy(), ref)
+    ref = np.zeros(8193)
+    lib.slice_smooth(dt, ref, 0.0, 2.5e-9)
+    got = torch.full((8193,), 7.0, dtype=torch.float64, device="cuda")
+    bm.slice_smooth(x, got, 0.0, 2.5e-9)
+    # as above
+    tol = n * 2.0 ** -(min(44, 60 - int(np.ceil(np.log2(max(n, 2)))))) + n * 2.0 ** -52 * ref.max()
+    assert np.max(np.abs(got.cpu().numpy() - ref)) <= max(tol, 1e-300)
+
+
 @pytest.mark.parametrize("n", SIZES)
 @pytest.mark.parametrize("shift", [0, 1])
 @pytest.mark.parametrize("lost", [None, "some", "all"])
