@@ -835,10 +835,14 @@ __global__ void __launch_bounds__(kAdjSliceBlock) adj_iv_kernel(AdjArgs a, int t
     }
 }
 
-// The pass's correlation: workgroup b sums corr[m] over turns b, b + grid, ...
-// into its row of `part`, for the entries that have a term (m < ns, then
-// m > n_fft - ns).  Once a pass (100 turns of 256 slices: 11 us, and 6.5 for
-// the rows' sum), where every turn's slice launch held it before.
+// The pass's correlation: workgroup (b, q) sums the q-th share of corr[m] over
+// turns b, b + grid, ... into row b of `part`, for the entries that have a term
+// (m < ns, then m > n_fft - ns).  Once a pass, where every turn's slice launch
+// held it before.  A turn's share of it is ns^2 products on one CU, so with
+// fewer turns than CUs the outputs are split over the others (corr_parts).
+// 256 slices: 4.7 us for 50 turns, 6.8 for 100 (one workgroup a turn 10.4 and
+// 10.6); 1024 slices: 9.1 us for one turn, 28 for 50, 64 for 100 (113, 116,
+// 119).
 __host__ __device__ __forceinline__ int corr_outputs(int ns, int n_fft) {
     const int hi0 = ns > n_fft - ns + 1 ? ns : n_fft - ns + 1;
     return ns + (n_fft - hi0);
@@ -848,6 +852,8 @@ __global__ void __launch_bounds__(kAdjSliceBlock) adj_corr_kernel(AdjArgs a, int
     extern __shared__ double sh[];
     const int ns = a.ns, n_out = corr_outputs(ns, a.n_fft), first = a.n_fft - (n_out - ns);
     double *lvs = sh, *p = sh + ns;
+    const int per = (n_out + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int o0 = (int)blockIdx.y * per, o1 = min(n_out, o0 + per);
     // kLanes lanes an output; an output's sum is added to by the same lane
     // over the turns
     for (int t = blockIdx.x; t < turns; t += gridDim.x) {
@@ -857,7 +863,7 @@ __global__ void __launch_bounds__(kAdjSliceBlock) adj_corr_kernel(AdjArgs a, int
             p[i] = a.prof[(size_t)t * ns + i];
         }
         __syncthreads();
-        for (int q = threadIdx.x; q < n_out * kLanes; q += blockDim.x) {
+        for (int q = o0 * kLanes + (int)threadIdx.x; q < o1 * kLanes; q += blockDim.x) {
             const int o = q / kLanes, r = q % kLanes;
             const int m = o < ns ? o : first + (o - ns);
             const double v = lanes_sum(circ_dot<1>(p, a.n_fft, ns, lvs, r, ns, -m));
@@ -882,10 +888,15 @@ __global__ void adj_corr_sum_kernel(const double *__restrict__ part, int rows, i
     corr[m] = v;
 }
 
-// Workgroups of the pass's correlation: a turn each, as many as there are CUs.
+// Workgroups of the pass's correlation: a turn each, as many as there are CUs,
+// and as many times over, at least a workgroup's 64 outputs each, as CUs are left.
 static int corr_rows(int turns) {
     const int cus = device_cu_count();
     return turns < cus ? turns : cus;
+}
+static int corr_parts(int rows, int n_out) {
+    const int most = (n_out + kAdjSliceOut - 1) / kAdjSliceOut, left = device_cu_count() / rows;
+    return left < most ? left : most;
 }
 
 // Workgroups of the slice-axis kernels: 64 outputs each.
@@ -1159,7 +1170,8 @@ static int enqueue_backward_map(Adjoint &j, int T, hipStream_t s) {
                                    t, !FUSE && t > 0);
         }
     }
-    hipLaunchKernelGGL(adj_corr_kernel, dim3(rows), dim3(kAdjSliceBlock),
+    const int parts = corr_parts(rows, corr_outputs(ns, (int)j.n_fft));
+    hipLaunchKernelGGL(adj_corr_kernel, dim3(rows, parts), dim3(kAdjSliceBlock),
                        sizeof(double) * 2 * (size_t)ns, s, a, T, j.d_corr_part);
     hipLaunchKernelGGL(adj_corr_sum_kernel, dim3((unsigned)((j.n_fft + 63) / 64)), dim3(64), 0, s,
                        j.d_corr_part, rows, ns, (int)j.n_fft, j.d_corr);

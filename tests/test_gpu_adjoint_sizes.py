@@ -24,7 +24,10 @@ KEYS = ("V", "phi", "R", "fr", "Q")
 @pytest.mark.parametrize("n,n_slices,every,turns", [
     (5001, 15, 3, 7), (5000, 16, 1, 5), (5001, 17, 4, 5), (1, 64, 2, 4), (20001, 255, 50, 6),
     (20000, 257, 4, 9), (20001, 511, 5, 6), (20001, 512, 5, 6), (20000, 513, 5, 6),
-    (20001, 1024, 3, 4), (2 * 262144 * 2 + 5, 64, 3, 4)])
+    (20001, 1024, 3, 4), (2 * 262144 * 2 + 5, 64, 3, 4),
+    # the pass's correlation over few turns: as many shares of its outputs as
+    # there are 64 of them, shares cut short, and two
+    (5001, 1024, 1, 1), (5001, 300, 2, 12), (5001, 100, 50, 100)])
 def test_profile_and_gradient_at_size_edges(n, n_slices, every, turns, map):
     """The forward profile to 1e-8 of its peak and the gradient to 1e-6 of
     the float64 CPU map's (the bars of the full-size tests): the piecewise
