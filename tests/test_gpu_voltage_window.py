@@ -16,9 +16,9 @@ from blond_amd.utils import bm  # noqa: E402
 from blond_amd.workloads import build_workload  # noqa: E402
 
 
-def _run(name, turns, peel, **kw):
+def _run(name, turns, peel, launch=None, **kw):
     w = build_workload(name, n_turns=turns + 1, **kw)
-    w.fused(1, max_peel=peel)
+    w.fused(1, max_peel=peel, **(launch or {}))
     w.fused(turns - 1)
     return [a.cpu().numpy() for a in (w.beam.dt, w.beam.dE, w.profile.n_macroparticles,
                                       w.tiv.induced_voltage)]
@@ -39,6 +39,17 @@ def test_same_bits_as_the_gathering_kernel(name, n_slices, n_fft, n, precision):
             assert np.array_equal(a, b)
     finally:
         bm.use_precision("double")
+
+
+# fewer threads stage the window, in more rounds and with the last round cut
+# short; at 20000 slices it starts at an odd bin
+@pytest.mark.parametrize("name,n_slices,n_fft", [("c2", 20000, 20000), ("c3", 65536, 131072)])
+@pytest.mark.parametrize("block,per_cu", [(64, 1), (256, 2), (512, 1)])
+def test_same_bits_at_other_launch_shapes(name, n_slices, n_fft, block, per_cu):
+    kw = dict(n_particles=300001, n_slices=n_slices, n_fft=n_fft,
+              launch=dict(block=block, blocks_per_cu=per_cu))
+    for a, b in zip(_run(name, 3, 0, **kw), _run(name, 3, 1, **kw)):
+        assert np.array_equal(a, b)
 
 
 def _turn_matches_oracle(w):
