@@ -321,6 +321,22 @@ __device__ __forceinline__ double bin_line(double b, double cut_left, double ste
     return ((b * step + cut_left) + ((b + 1.0) * step + cut_left)) * 0.5;
 }
 
+// Whether the bin centres of turn t's table are on that line: a launch that
+// forms the table sets flags[t & 1] where one is not, and clears the next
+// turn's word (read last by turn t - 1's particles).
+struct BinLine {
+    int *flags;  // nullptr: not asked for
+    double cut_left, step;
+    __device__ __forceinline__ bool off(int b, double bc) const {
+        return flags && bc != bin_line((double)b, cut_left, step);
+    }
+    // by every thread of the launch, `clears` in one of them
+    __device__ __forceinline__ void put(bool any_off, int t, bool clears) const {
+        if (any_off) flags[t & 1] = 1;
+        if (flags && clears) flags[(t + 1) & 1] = 0;
+    }
+};
+
 // A table entry as stored: a (slope, intercept) pair of doubles, or with f32
 // of floats, which hold the single build's FP32 values exactly and halve the
 // bytes the kick gathers (the table then holds float2 entries; its

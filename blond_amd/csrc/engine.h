@@ -51,8 +51,10 @@ struct Engine {
     double charge = 1.0;
     double *d_rf = nullptr, *d_acc = nullptr;
     DriftCoeffs<double> *d_drift = nullptr;
-    int *d_base = nullptr;         // [0] turn base, [1..2] pending flags of the count buffers
-    int *d_bc_off = nullptr;       // [kWave]: whether bin centres are off the cuts' line
+    // [0] turn base, [1..2] pending flags of the count buffers, [3..4] by turn
+    // parity: whether the turn's table has a bin centre off the cuts' line
+    int *d_base = nullptr;
+    int *line_flags() const { return d_base + 3; }
     void *d_sink = nullptr;        // kSinkBytes: the particle kernels' store target for idle lanes
     int host_turn = 0;             // mirror of the turn base, kept by set_turn/track
     // slicing: counts double buffered by turn parity
@@ -233,8 +235,7 @@ struct Engine {
     int launch_window_turn(hipStream_t s, int off, bool interp, const KernelEvents &ev);
     int ensure_partials();
     bool near_kernel(int imode, bool hist, int ldsh) const;
-    int check_bin_line(hipStream_t s);
-    double bin_step() const { return (cut_right - cut_left) / (double)n_slices; }
+    BinLine bin_line_args() const;
     // whether the u16-pair rows are stored transposed for the four-step
     // transform's first pass, which then sums them itself (no reduction
     // launch); shift = log2 M2 and lshift = log2 of the words per column

@@ -88,12 +88,10 @@ struct TurnArgs {
     // interpolation table from L2: entries [tw_lo, tw_lo + tw_n) staged in
     // LDS after the histogram (tw_n 0: none); FP64 NEAR kernels stage the
     // tw_n + 1 voltages under them, and form an entry from two of them and the
-    // bin centre on a line of spacing `step` from the left cut, unless a word
-    // of bc_off says that the bin centres are not on it
+    // bin centre on `line`, unless its flag says that the bin centres are not on it
     int tw_lo, tw_n;
     const double *volt;
-    double step;
-    const int *bc_off;                 // [kWave]
+    BinLine line;
     // bunch moments of the coordinates after the drift: workgroup b writes
     // sum(dt - shift_t), sum((dt - shift_t)^2), sum(dE - shift_e),
     // sum((dE - shift_e)^2) of its particles to stats[(t + 1) * grid + b]
@@ -233,19 +231,6 @@ typedef Double2 Double2Any __attribute__((aligned(8)));
 template <typename T> struct TabEntry { using type = double2; };
 template <> struct TabEntry<float> { using type = float2; };
 
-// bc_off[b] = 1 where a bin centre of workgroup b's share (grid: kWave) is not
-// the middle of the edges b step + cut_left and (b + 1) step + cut_left, as
-// numpy's linspace and mean give them
-__global__ void __launch_bounds__(1024) bin_line_kernel(const double *__restrict__ bc, int n_tab,
-                                                        double cut_left, double step,
-                                                        int *__restrict__ bc_off) {
-    int off = 0;
-    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < n_tab; b += gridDim.x * blockDim.x)
-        off |= bc[b] != bin_line(b, cut_left, step);
-    off = __syncthreads_or(off);
-    if (threadIdx.x == 0) bc_off[blockIdx.x] = off;
-}
-
 // 16 (double) or 8 (float) bytes of a pair of coordinates through a buffer
 // descriptor: an offset past its end loads zeros and stores nothing
 template <typename V2, int POLICY>
@@ -350,7 +335,7 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         ea = reinterpret_cast<const V2 *>(dE)[clamp(i_first)];
     }
     constexpr bool kVoltWindow = NEAR && sizeof(T) == 8;
-    const bool line_off = kVoltWindow && __any(a.bc_off[threadIdx.x % kWave]);
+    const bool line_off = kVoltWindow && a.line.flags[t & 1] != 0;
     // the histogram words (with windowed rows, the window's); the padded
     // layout adds one word per 2^part_shift (none when 31)
     const int hwords = (HIST && LDSH) ? ((LDSH == 2 && a.win_bins) ? a.win_bins / 2
@@ -397,7 +382,7 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
     T q_charge = a.charge, q_acc = acc, q_cl = a.cut_left, q_ibw = a.inv_bw;
     T q_ntab = (T)a.n_tab, q_ns = (T)a.n_slices, q_bc0 = bc0, q_tibw = ibw;
     int q_twlo = a.tw_lo, q_twn = line_off ? 0 : a.tw_n, q_wlo = a.win_lo, q_wn = a.win_bins;
-    const T q_step = (T)a.step;
+    const T q_step = (T)a.line.step;
     uint64_t q_tabp = (uint64_t)a.tab, q_cntp = (uint64_t)a.cnt_out;
     auto pin_constants = [&]() {
         asm volatile("" : "+v"(q_charge), "+v"(q_acc), "+v"(q_cl), "+v"(q_ibw));
@@ -898,9 +883,7 @@ void Engine::release() {
     (void)hipFree(d_drift);
     (void)hipFree(d_base);
     (void)hipFree(d_sink);
-    (void)hipFree(d_bc_off);
     d_sink = nullptr;
-    d_bc_off = nullptr;
     (void)hipFree(d_counts);
     (void)hipFree(d_table);
     (void)hipFree(d_Z);
@@ -974,9 +957,9 @@ int Engine::init(int64_t n_particles, int n_rf_, int n_turns_, int solver_) {
     BLMI_HIP_TRY(hipMalloc(&d_drift, sizeof(DriftCoeffs<double>) * (size_t)(n_turns + 1)));
     BLMI_HIP_TRY(hipMalloc(&d_trev, sizeof(double) * (size_t)(n_turns + 1)));
     // d_base[0] = turn base, d_base[1..2] = turn held by each count buffer (-1: none)
-    BLMI_HIP_TRY(hipMalloc(&d_base, sizeof(int) * 4));
+    BLMI_HIP_TRY(hipMalloc(&d_base, sizeof(int) * 5));
     BLMI_HIP_TRY(hipMalloc(&d_sink, kSinkBytes));
-    BLMI_HIP_TRY(hipMemset(d_base, 0, sizeof(int)));
+    BLMI_HIP_TRY(hipMemset(d_base, 0, sizeof(int) * 5));
     BLMI_HIP_TRY(hipMemset(d_base + 1, 0xff, sizeof(int) * 2));
     BLMI_HIP_TRY(hipStreamCreateWithFlags(&own_stream, hipStreamNonBlocking));
     BLMI_HIP_TRY(hipEventCreateWithFlags(&ev_in, hipEventDisableTiming));
@@ -1235,6 +1218,7 @@ int Engine::set_turn(int turn) {
         BLMI_HIP_TRY(hipMemset(d_counts, 0,
                                sizeof(unsigned) * 2 * (size_t)groups * (size_t)n_slices));
     BLMI_HIP_TRY(hipMemset(d_base + 1, 0xff, sizeof(int) * 2));
+    BLMI_HIP_TRY(hipMemset(line_flags(), 0, sizeof(int) * 2));
     return BLMI_OK;
 }
 
@@ -1258,9 +1242,12 @@ int Engine::launch_block() const {
 
 // The u16-row intensity kernels take buffer descriptors (turn_kernel NEAR)
 // while every offset of a launch, two strides past the end included, fits 32
-// bits, the counts are not merged and the table is the induced voltage's own.
+// bits, the counts are not merged and the table is the induced voltage's own,
+// formed by a launch that compares the bin centres with the cuts' line (the
+// four-step transform's last, or the wake step's).
 bool Engine::near_kernel(int imode, bool hist, int ldsh) const {
     if (imode != 1 || !hist || ldsh != 2 || !intensity || interp_rf || max_peel > 0) return false;
+    if (have_conv && method != 2) return false;
     int grid = 0;
     size_t lds = 0;
     const int block = launch_block();
@@ -1269,20 +1256,18 @@ bool Engine::near_kernel(int imode, bool hist, int ldsh) const {
     return (n / 2 + 4 * (int64_t)grid * block) * pair < (int64_t)1 << 32;
 }
 
-// Words of bc_off for the voltage window, from the bin centres as they are now.
-int Engine::check_bin_line(hipStream_t s) {
-    if (f32 || !intensity || ordered() || n_slices < 2) return BLMI_OK;
+// What the launch that forms the table compares the bin centres with, where
+// the particle kernel takes the voltage window: that launch reads them anyway.
+// (A comparison of its own in every track() call: 65536 slices, 1e6
+// macroparticles, track(1) 68.5 us in place of 61.8.)
+BinLine Engine::bin_line_args() const {
+    BinLine l{nullptr, cut_left, (cut_right - cut_left) / (double)n_slices};
     int grid = 0;
     size_t lds = 0;
-    const int mode = hist_layout(launch_block(), &grid, &lds);
-    if (mode != 2 || !near_kernel(1, d_counts != nullptr, mode)) return BLMI_OK;
-    if (!d_bc_off) {
-        invalidate_graph();
-        BLMI_HIP_TRY(hipMalloc(&d_bc_off, sizeof(int) * kWave));
-    }
-    hipLaunchKernelGGL(bin_line_kernel, dim3(kWave), dim3(1024), 0, s, bc, n_slices - 1, cut_left,
-                       bin_step(), d_bc_off);
-    return blmi_check_launch("bin_line");
+    if (!f32 && !ordered() && d_counts &&
+        near_kernel(1, true, hist_layout(launch_block(), &grid, &lds)))
+        l.flags = line_flags();
+    return l;
 }
 
 int Engine::hist_layout(int block, int *grid_out, size_t *lds_out) const {
@@ -1646,8 +1631,7 @@ static int launch_turn_t(const Engine &e, T *x, T *de, const T *rf, const T *acc
     const bool near = e.near_kernel(imode, hist, ldsh);
     if (near) {
         a.volt = e.volt;
-        a.step = e.bin_step();
-        a.bc_off = e.d_bc_off;
+        a.line = e.bin_line_args();
     }
     if (imode == 1 && hist && ldsh == 2 && a.n_tab > 0) {
         // the LDS the u16 rows leave holds a window of the table, centred on
@@ -1773,6 +1757,7 @@ InducedArgs Engine::induced_args(int off) const {
     ia.tab = reinterpret_cast<double2 *>(d_table);
     ia.tab_params = d_table + 2 * n_slices;
     ia.f32 = f32 ? 1 : 0;
+    ia.line = bin_line_args();
     int ps = 31, pl = 0, m1lo = 0;
     ia.part = nullptr;
     ia.cnt_out = nullptr;
@@ -2003,6 +1988,7 @@ WakeArgs Engine::wake_args(int off) const {
     a.volt = volt;
     a.tab = reinterpret_cast<double2 *>(d_table);
     a.tab_params = d_table + 2 * n_slices;
+    a.line = bin_line_args();
     return a;
 }
 
@@ -2236,8 +2222,6 @@ int Engine::time_kernels(int turns, hipStream_t user, float *ms_induced, float *
         prc = launch_mtw_load(d_base, d_mem, d_mem + n_mem, n_mem, mem_user, own_stream);
         if (prc) return prc;
     }
-    prc = check_bin_line(own_stream);
-    if (prc) return prc;
     std::vector<hipEvent_t> ev(4 * (size_t)turns, nullptr);
     for (auto &x : ev) BLMI_HIP_TRY(hipEventCreate(&x));
     int rc = BLMI_OK;
@@ -2310,8 +2294,6 @@ int Engine::track(int turns, hipStream_t user, bool use_graph) {
         prc = launch_mtw_load(d_base, d_mem, d_mem + n_mem, n_mem, mem_user, own_stream);
         if (prc) return prc;
     }
-    prc = check_bin_line(own_stream);
-    if (prc) return prc;
     int done = 0;
     int rc = BLMI_OK;
     if (use_graph && turns >= chunk) {

@@ -64,6 +64,7 @@ struct InducedArgs {
     double2 *tab;
     double *tab_params;
     int f32;          // table in the reference's single-precision arithmetic
+    BinLine line;     // four-step method: the table's bin centres against the cuts' line
     // four-step method: the profile as the sum of part_rows u16-pair rows
     // stored transposed (column m2's word m1 of row r at
     // part[(m2 part_rows + r) 2^part_lshift + m1]); nullptr: the counts

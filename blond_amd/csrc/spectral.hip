@@ -1425,6 +1425,7 @@ __global__ void __launch_bounds__(kColThreads) fft2_c_kernel(InducedArgs a, int 
         a.tab_params[0] = a.bc[0];
         a.tab_params[1] = inv_bw;
     }
+    bool off = false;
     for (int j = threadIdx.x; j < cols * M1; j += kColThreads) {
         const int c = j % cols, m1 = j / cols;
         const int m = M2 * m1 + c0 + c;
@@ -1434,6 +1435,7 @@ __global__ void __launch_bounds__(kColThreads) fft2_c_kernel(InducedArgs a, int 
         if (2 * m + 1 < a.n_out) a.volt[2 * m + 1] = v1;
         if (a.tab && 2 * m < ns - 1) {
             const double b0 = one ? bc_pre[0] : a.bc[2 * m];
+            off |= a.line.off(2 * m, b0);
             store_interp_entry(a.tab, 2 * m, interp_entry(v0, v1, b0, a.charge, inv_bw, a.f32),
                                a.f32);
             if (2 * m + 1 < ns - 1) {
@@ -1442,11 +1444,14 @@ __global__ void __launch_bounds__(kColThreads) fft2_c_kernel(InducedArgs a, int 
                                    : buf[cols * ld + (last ? m1 + 1 : m1)];
                 const double v2 = -(a.scale * (un.x * fct));
                 const double b1 = one ? bc_pre[1] : a.bc[2 * m + 1];
+                off |= a.line.off(2 * m + 1, b1);
                 store_interp_entry(a.tab, 2 * m + 1,
                                    interp_entry(v1, v2, b1, a.charge, inv_bw, a.f32), a.f32);
             }
         }
     }
+    if (a.line.flags)
+        a.line.put(off, *a.turn_base + a.turn_off, blockIdx.x == 0 && threadIdx.x == 0);
 }
 
 static bool factor_list(int L, int *radix, int &n) {

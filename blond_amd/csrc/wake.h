@@ -165,6 +165,7 @@ struct WakeArgs {
     double *volt;
     double2 *tab;           // (slope, intercept) per bin, tab_params = (bc[0], inv_bw)
     double *tab_params;
+    BinLine line;           // wake_finish: the table's bin centres against the cuts' line
 };
 int launch_wake_finish(const WakeArgs &a, hipStream_t s, const KernelEvents &ev = KernelEvents());
 // memory[(*turn_base) & 1] -> out[n_mem] (publish the current memory)

@@ -126,6 +126,7 @@ __global__ void __launch_bounds__(kWakeBlock) wake_finish_kernel(WakeArgs a) {
         return v;
     };
 
+    bool off = false;
     if (i < a.n_mem) mem_out[i] = mem_at(i);
     if (i < ns) {
         if (from_counts) {
@@ -144,8 +145,10 @@ __global__ void __launch_bounds__(kWakeBlock) wake_finish_kernel(WakeArgs a) {
             const double vn = total_at((int)i + 1);
             const double k = a.charge * (vn - vi) * inv_bw;
             a.tab[i] = make_double2(k, (a.charge * vi - a.bc[i] * k) + 0.0);
+            off = a.line.off((int)i, a.bc[i]);
         }
     }
+    a.line.put(off, t, i == 0);
 }
 
 int launch_wake_finish(const WakeArgs &a, hipStream_t s, const KernelEvents &ev) {

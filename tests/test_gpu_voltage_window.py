@@ -13,7 +13,7 @@ if not torch.cuda.is_available():  # pragma: no cover
     pytest.skip("no GPU", allow_module_level=True)
 
 from blond_amd.utils import bm  # noqa: E402
-from blond_amd.workloads import build_workload  # noqa: E402
+from blond_amd.workloads import build_wake_workload, build_workload  # noqa: E402
 
 
 def _run(name, turns, peel, launch=None, **kw):
@@ -68,7 +68,63 @@ def test_bin_centres_off_the_line_use_the_table():
     _turn_matches_oracle(w)
     bc = w.profile.bin_centers
     step = float(w.profile.bin_size)
+    line = bc.clone()
     for at in (32768, 31000):
         bc[at:at + 1000] += 0.1 * step
         _turn_matches_oracle(w)
-    bc[32768:33768] -= 0.1 * step
+    bc.copy_(line)
+    _turn_matches_oracle(w)
+
+
+def _both(build):
+    """Two workloads of the same bunch, one tracked by each kernel."""
+    return [(build(), dict(max_peel=peel)) for peel in (0, 1)]
+
+
+def _same(pair):
+    (a, _), (b, _) = pair
+    for x, y in ((a.beam.dt, b.beam.dt), (a.beam.dE, b.beam.dE),
+                 (a.profile.n_macroparticles, b.profile.n_macroparticles),
+                 (a.tiv.induced_voltage, b.tiv.induced_voltage)):
+        assert torch.equal(x, y)
+
+
+def _builds():
+    yield lambda: build_workload("c2", n_particles=60001, n_turns=40, n_slices=20000,
+                                 n_fft=20000, intensity=1e13)
+    yield lambda: build_workload("c3", n_particles=60001, n_turns=40, n_slices=65536,
+                                 n_fft=131072, intensity=1e13)
+    # the wake step forms the table: a multi-turn memory, an inductive source
+    # alone (no transform) and beside a convolution
+    for kind in ("mtw", "zovern", "mixed"):
+        yield lambda kind=kind: build_wake_workload(kind, n_particles=60001, n_turns=40,
+                                                    n_slices=20000, memory_turns=2)
+
+
+@pytest.mark.parametrize("build", _builds(), ids=["c2", "c3", "mtw", "zovern", "mixed"])
+def test_bin_centres_on_and_off_the_line(build):
+    """The same bits as the gathering kernel while centres leave the line and
+    come back between calls of one, two and three turns: the first, one
+    inside the window and the last of the table's, and the one past it, which
+    only scales the table; then the program started again."""
+    pair = _both(build)
+    ns = pair[0][0].profile.n_slices
+    line = [w.profile.bin_centers.clone() for w, _ in pair]
+    step = float(pair[0][0].profile.bin_size)
+    for turns, moved in ((1, None), (2, ns // 2), (1, ns // 2 + 7), (3, None), (1, 0), (1, None),
+                         (2, ns - 2), (1, None), (1, None), (3, ns - 1), (2, None)):
+        for (w, kw), l in zip(pair, line):
+            w.profile.bin_centers.copy_(l)
+            if moved is not None:
+                w.profile.bin_centers[moved] += 0.1 * step
+            w.fused(turns, **kw)
+        _same(pair)
+    if getattr(pair[0][0].tiv.induced_voltage_list[0], "multi_turn_wake", False):
+        return  # the memory belongs to the turns before
+    for w, kw in pair:
+        w.profile.bin_centers[ns // 2] += 0.1 * step
+        w.fused(1)
+        w.rf.counter[0] = 0
+        w.profile.bin_centers.copy_(line[0])
+        w.fused(3)
+    _same(pair)
