@@ -272,6 +272,9 @@ constexpr int kBufferFlags = 0x00027000;
 // rate of an in-place copy: 41 and 175 us); FP32, addresses only, 1e7 45.9 ->
 // 44.5 us.  Measured the same: two pairs more in flight, gathers issued before
 // the stores, part of a 3e7 bunch kept in the last-level cache.
+// Where bin centres are off the line the window holds entries, half as many,
+// as in the general kernel: 1e7 macroparticles 65.4 us, 3e7 298 (76.3 and 335
+// with every entry gathered).
 template <typename T, int SOLVER, int INTERP, bool HIST, int LDSH, bool PUBLISH, bool NT = false,
           bool NEAR = false>
 __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__restrict__ dE,
@@ -349,21 +352,23 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
     TabE *ltab = reinterpret_cast<TabE *>(lds_hist + ((lwords + 3) & ~3));
     constexpr bool kTabWindow = INTERP == 1 && HIST && LDSH == 2;
     const bool tw_on = kTabWindow && a.tw_n > 0;
+    // bin centres off the line: the table's entries in the voltages' place, half
+    // as many around the same bin
+    const int tw_n = line_off ? a.tw_n / 2 : a.tw_n;
+    const int tw_lo = line_off ? a.tw_lo + tw_n / 2 : a.tw_lo;
     if ((HIST && LDSH) || INTERP == 2) {
         for (int b = threadIdx.x; b < lwords; b += blockDim.x) lds_hist[b] = 0u;
         if (INTERP == 2)
             for (int k = threadIdx.x; k < a.n_tab; k += blockDim.x) ltab[k] = gtab[k];
-        if (tw_on) {
-            if constexpr (kVoltWindow) {
-                // two a load, as an entry is (tw_n is even, tw_lo may be odd);
-                // one a load: 0.7 us more at 1024 threads, 6 at 256
-                const double *v = a.volt + a.tw_lo;
-                for (int k = threadIdx.x; k < a.tw_n / 2; k += blockDim.x)
-                    reinterpret_cast<Double2 *>(ltab)[k] = reinterpret_cast<const Double2Any *>(v)[k];
-                if (threadIdx.x == 0) reinterpret_cast<double *>(ltab)[a.tw_n] = v[a.tw_n];
-            } else {
-                for (int k = threadIdx.x; k < a.tw_n; k += blockDim.x) ltab[k] = gtab[a.tw_lo + k];
-            }
+        if (tw_on && kVoltWindow && !line_off) {
+            // two a load, as an entry is (tw_n is even, tw_lo may be odd);
+            // one a load: 0.7 us more at 1024 threads, 6 at 256
+            const double *v = a.volt + tw_lo;
+            for (int k = threadIdx.x; k < tw_n / 2; k += blockDim.x)
+                reinterpret_cast<Double2 *>(ltab)[k] = reinterpret_cast<const Double2Any *>(v)[k];
+            if (threadIdx.x == 0) reinterpret_cast<double *>(ltab)[tw_n] = v[tw_n];
+        } else if (tw_on) {
+            for (int k = threadIdx.x; k < tw_n; k += blockDim.x) ltab[k] = gtab[tw_lo + k];
         }
     }
     __syncthreads();  // the LDS set-up, and the sine's coefficient table
@@ -381,7 +386,7 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
     // v_readlane at every use)
     T q_charge = a.charge, q_acc = acc, q_cl = a.cut_left, q_ibw = a.inv_bw;
     T q_ntab = (T)a.n_tab, q_ns = (T)a.n_slices, q_bc0 = bc0, q_tibw = ibw;
-    int q_twlo = a.tw_lo, q_twn = line_off ? 0 : a.tw_n, q_wlo = a.win_lo, q_wn = a.win_bins;
+    int q_twlo = tw_lo, q_twn = tw_n, q_wlo = a.win_lo, q_wn = a.win_bins;
     const T q_step = (T)a.line.step;
     uint64_t q_tabp = (uint64_t)a.tab, q_cntp = (uint64_t)a.cnt_out;
     auto pin_constants = [&]() {
@@ -391,7 +396,8 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         if (kTabWindow) asm volatile("" : "+v"(q_twlo), "+v"(q_twn), "+v"(q_tabp));
         if (HIST && LDSH == 2) asm volatile("" : "+v"(q_wlo), "+v"(q_wn), "+v"(q_cntp));
     };
-    auto gather = [&](T x) -> Tab {
+    // volts: the window holds voltages
+    auto gather = [&](T x, auto volts) -> Tab {
         Tab g{TabE{}, false};
         if (INTERP) {
             const T f = floor((x - q_bc0) * q_tibw);
@@ -407,7 +413,7 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
                 TabE kg;
                 kg.x = kv.x;
                 kg.y = kv.y;
-                if constexpr (kVoltWindow) {
+                if constexpr (decltype(volts)::value) {
                     g.k = kg;  // finish() reads the window itself
                 } else {
                     const TabE kl = ltw[intw ? kw : 0];
@@ -421,11 +427,11 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
     };
     // the rest of the turn of one particle given its table entry; the sums
     // keep the order e + interp + rf
-    auto finish = [&](T &x, T &e, const Tab &g, auto nrf) -> int {
+    auto finish = [&](T &x, T &e, const Tab &g, auto nrf, auto volts) -> int {
         constexpr int NRF = decltype(nrf)::value;
         T v0 = T(0), v1 = T(0), f0 = T(0);
         bool win = false;
-        if constexpr (kVoltWindow) {
+        if constexpr (decltype(volts)::value) {
             f0 = floor((x - q_bc0) * q_tibw);
             const int kw = (int)f0 - q_twlo;
             win = g.in && (unsigned)kw < (unsigned)q_twn;
@@ -436,7 +442,7 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         const T rf = rfp.template kick_tab<NRF>(x, q_charge, q_acc, stab);
         if (INTERP) {
             T slope = (T)g.k.x, cut = (T)g.k.y;
-            if constexpr (kVoltWindow) {
+            if constexpr (decltype(volts)::value) {
                 // interp_entry on the bin's line centre
                 const double2 k = interp_entry(v0, v1, bin_line(f0, q_cl, q_step), q_charge,
                                                q_tibw, false);
@@ -494,7 +500,9 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         __builtin_amdgcn_make_buffer_rsrc((void *)dE, 0, bytes, kBufferFlags);
     constexpr int kPolicy = NT ? kPolicyNt : 0;
     const unsigned stride_bytes = (unsigned)stride * (unsigned)sizeof(V2);
-    // one copy of the particle loop per RF-system count (see with_rf_count)
+    // one copy of the particle loop per RF-system count (see with_rf_count) and
+    // kind of window
+    auto turn = [&](auto volts) {
     with_rf_count(a.n_rf, [&](auto nrf) {
     if constexpr (!NEAR) {
         rfp.template pin<decltype(nrf)::value>();
@@ -506,8 +514,8 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
     auto pair = [&](auto more, V2 &x, V2 &e, Tab &g0, Tab &g1, const V2 &xo, Tab &go0,
                     Tab &go1, int64_t i, unsigned off) {
         const bool own = NEAR ? off < (unsigned)bytes : i < n2;
-        int b0 = finish(x.x, e.x, g0, nrf);
-        int b1 = finish(x.y, e.y, g1, nrf);
+        int b0 = finish(x.x, e.x, g0, nrf, volts);
+        int b1 = finish(x.y, e.y, g1, nrf, volts);
         if constexpr (NEAR) {
             buffer_store_pair<V2, kPolicy>(rx, off, x);
             buffer_store_pair<V2, kPolicy>(re, off, e);
@@ -536,8 +544,8 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
             b0 = b1 = -1;
         }
         if constexpr (decltype(more)::value) {
-            go0 = gather(xo.x);
-            go1 = gather(xo.y);
+            go0 = gather(xo.x, volts);
+            go1 = gather(xo.y, volts);
             if constexpr (NEAR) {
                 x = buffer_load_pair<V2, kPolicy>(rx, off + 2 * stride_bytes);
                 e = buffer_load_pair<V2, kPolicy>(re, off + 2 * stride_bytes);
@@ -560,7 +568,7 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         count(b1);
     };
     if (iters > 0) {
-        Tab ga0 = gather(xa.x), ga1 = gather(xa.y), gb0{}, gb1{};
+        Tab ga0 = gather(xa.x, volts), ga1 = gather(xa.y, volts), gb0{}, gb1{};
         xb = reinterpret_cast<const V2 *>(dt)[clamp(i_first + stride)];
         eb = reinterpret_cast<const V2 *>(dE)[clamp(i_first + stride)];
         // both slots every iteration, no exit between them (a branch there
@@ -582,8 +590,8 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         int b = -1;
         if (threadIdx.x == 0) {
             T x = dt[n - 1], e = dE[n - 1];
-            const Tab g = gather(x);
-            b = finish(x, e, g, nrf);
+            const Tab g = gather(x, volts);
+            b = finish(x, e, g, nrf, volts);
             dt[n - 1] = x;
             dE[n - 1] = e;
             if (a.stats) moment(x, e);
@@ -591,6 +599,15 @@ __global__ void __launch_bounds__(1024) turn_kernel(T *__restrict__ dt, T *__res
         count(b);
     }
     });
+    };
+    if constexpr (kVoltWindow) {
+        if (line_off)
+            turn(std::false_type{});
+        else
+            turn(std::true_type{});
+    } else {
+        turn(std::false_type{});
+    }
     if (a.stats) stats_flush(st, a.stats + ((size_t)(t + 1) * gridDim.x + blockIdx.x) * 4);
     if (HIST && LDSH) {
         __syncthreads();

@@ -52,6 +52,23 @@ def test_same_bits_at_other_launch_shapes(name, n_slices, n_fft, block, per_cu):
         assert np.array_equal(a, b)
 
 
+# the window of entries where centres are off the line: 20000 slices (from an
+# odd bin) and 65536, no pair, one and an odd number of them a thread, and
+# fewer threads to stage it
+@pytest.mark.parametrize("name,n_slices,n_fft", [("c2", 20000, 20000), ("c3", 65536, 131072)])
+@pytest.mark.parametrize("n,block", [(1, 1024), (300001, 1024), (300001, 64),
+                                     (4 * 262144 + 3, 1024)])
+def test_same_bits_off_the_line(name, n_slices, n_fft, n, block):
+    out = []
+    for peel in (0, 1):
+        w = build_workload(name, n_particles=n, n_turns=4, n_slices=n_slices, n_fft=n_fft)
+        w.profile.bin_centers[n_slices // 3::2] += 0.1 * float(w.profile.bin_size)
+        w.fused(3, max_peel=peel, block=block)
+        out.append((w.beam.dt, w.beam.dE, w.profile.n_macroparticles, w.tiv.induced_voltage))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
 def _turn_matches_oracle(w):
     ref = orc.track(w.oracle_copy(), 1)
     w.fused(1)
