@@ -662,9 +662,26 @@ int blmi_engine_set_launch(void *h, int block, int blocks_per_cu, int graph_chun
     BLMI_REQUIRE(blocks_per_cu >= 1 && blocks_per_cu <= 64, "engine: blocks_per_cu in [1, 64]");
     BLMI_REQUIRE(graph_chunk >= 1 && graph_chunk <= 1000, "engine: graph_chunk in [1, 1000]");
     e->block_size = block;
+    e->block_auto = false;
     e->blocks_per_cu = blocks_per_cu;
     e->graph_chunk = graph_chunk;
     e->invalidate_graph();
+    return BLMI_OK;
+}
+
+int blmi_engine_set_auto_block(void *h, int on) {
+    Engine *e = reinterpret_cast<Engine *>(h);
+    BLMI_REQUIRE(e, "engine: null handle");
+    e->block_auto = on != 0;
+    e->invalidate_graph();
+    return BLMI_OK;
+}
+
+int blmi_engine_get_launch(void *h, int *block, int *blocks_per_cu) {
+    Engine *e = reinterpret_cast<Engine *>(h);
+    BLMI_REQUIRE(e && block && blocks_per_cu, "engine: null argument");
+    *block = e->launch_block();
+    *blocks_per_cu = e->blocks_per_cu;
     return BLMI_OK;
 }
 

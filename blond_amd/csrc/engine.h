@@ -152,8 +152,9 @@ struct Engine {
     double *d_zero_acc = nullptr;       // [n_turns + 1] zeros
     // launch shape (tunable)
     int block_size = 1024;
+    bool block_auto = true;        // block_size not given: less for small bunches
     int blocks_per_cu = 1;
-    int launch_block() const;      // the workgroup size launched: block_size or less
+    int launch_block() const;      // the workgroup size launched
     // plain tracking: at most this many turns per particle-kernel launch
     // (the particles stay in registers between them; 1 = a launch a turn)
     int turn_block = kTurnBlockDefault;

@@ -1244,8 +1244,9 @@ int Engine::get_turn(int *turn) {
     return BLMI_OK;
 }
 
-// The particle kernels' workgroup: the configured size, halved down to 256
-// threads while a thread still takes at most two pairs, so that a small bunch
+// The particle kernels' workgroup: the size the caller gave, or else 1024
+// threads, halved down to 256 while a thread still takes at most two pairs, so
+// that a small bunch
 // spreads over all CUs (moderate slice counts: with few threads the table's
 // staging and the histogram's clearing would dominate).  Turn kernel with 500
 // slices, 1024 threads against this: 5e4 macroparticles 6.4 / 5.1 us, 2e5 7.0 /
@@ -1253,7 +1254,7 @@ int Engine::get_turn(int *turn) {
 int Engine::launch_block() const {
     const int64_t wgs = (int64_t)device_cu_count() * blocks_per_cu, pairs = (n + 1) / 2;
     int b = block_size;
-    while (n_slices <= kSmallBlockSlices && b >= 512 && pairs <= wgs * b) b /= 2;
+    while (block_auto && n_slices <= kSmallBlockSlices && b >= 512 && pairs <= wgs * b) b /= 2;
     return b;
 }
 

@@ -139,9 +139,14 @@ def wake_setup(tiv, n_turns: int):
     return (mtw[0] if mtw else None), coef, mode
 
 
+class _DefaultBlock(int):
+    """The workgroup size nobody asked for: the engine may take a smaller one
+    (a small bunch of at most 1024 slices); a size that is given is kept."""
+
+
 class FusedTracker:
     def __init__(self, tracker, profile=None, total_induced_voltage=None, use_graph=True,
-                 block=1024, blocks_per_cu=1, graph_chunk=50, groups=0, max_peel=0,
+                 block=_DefaultBlock(1024), blocks_per_cu=1, graph_chunk=50, groups=0, max_peel=0,
                  method=None, sort_every=0, statistics=False, monitor=None, turn_block=25):
         import torch
 
@@ -200,6 +205,8 @@ class FusedTracker:
             self._setup_interpolation()
         _lib.call("blmi_engine_set_launch", self._h, int(block), int(blocks_per_cu),
                   int(graph_chunk))
+        if isinstance(block, _DefaultBlock):
+            _lib.call("blmi_engine_set_auto_block", self._h, 1)
         # plain turns: up to turn_block turns a launch (1: a launch a turn)
         _lib.call("blmi_engine_set_turn_block", self._h, int(turn_block))
         _lib.call("blmi_engine_set_hist", self._h, int(groups), int(max_peel))

@@ -295,8 +295,12 @@ int blmi_engine_get_programs(void *engine, int turn0, int turns, double *rf_host
 int blmi_engine_set_statistics(void *engine, int enable, double shift_dt, double shift_dE);
 int blmi_engine_get_statistics(void *engine, int turn0, int turns, double *moments_host);
 /* Launch shape of the particle kernel (block in {64..1024}, workgroups per CU)
- * and the number of turns per captured graph. */
+ * and the number of turns per captured graph.  An engine whose block was never
+ * set, or which is told so by set_auto_block afterwards, halves it for a small
+ * bunch of at most 1024 slices; get_launch gives the shape in use. */
 int blmi_engine_set_launch(void *engine, int block, int blocks_per_cu, int graph_chunk);
+int blmi_engine_set_auto_block(void *engine, int on);
+int blmi_engine_get_launch(void *engine, int *block, int *blocks_per_cu);
 /* Plain tracking (no intensity effects, statistics, phase loop,
  * interpolation table or sort, at most 65536/4 slices' u32 histogram): up to
  * max_turns turns (rounded down to odd) in one particle-kernel launch, the

@@ -53,3 +53,27 @@ def test_intensity_turn_launch_shapes(name, block, per_cu, groups):
     sc = np.abs(ref["dE"]).max()
     np.testing.assert_allclose(host(w.beam.dE), ref["dE"], rtol=0, atol=1e-12 * sc)
     np.testing.assert_allclose(host(w.beam.dt), ref["dt"], rtol=1e-12, atol=0)
+
+
+def test_a_given_block_is_kept():
+    """5000 macroparticles on 100 slices: 256 threads where nothing was given,
+    else what was, the default's value among it."""
+    for given, want in (({}, 256), (dict(block=1024), 1024), (dict(block=512), 512),
+                        (dict(block=64, blocks_per_cu=2), 64)):
+        for name in ("c1", "c2"):
+            w = build_workload(name, n_particles=5000, n_turns=4, n_slices=100,
+                               **({} if name == "c1" else dict(n_fft=200)))
+            assert _shape(w.fused(2, **given)) == (want, given.get("blocks_per_cu", 1))
+    # many macroparticles or many slices: the default's full size
+    for kw in (dict(n_particles=1_100_000, n_slices=100), dict(n_particles=5000, n_slices=2000)):
+        assert _shape(build_workload("c1", n_turns=4, **kw).fused(1)) == (1024, 1)
+
+
+def _shape(ft):
+    import ctypes as ct
+
+    from blond_amd import _lib
+
+    block, per_cu = ct.c_int(), ct.c_int()
+    _lib.call("blmi_engine_get_launch", ft._h, ct.byref(block), ct.byref(per_cu))
+    return block.value, per_cu.value
