@@ -18,7 +18,10 @@ namespace blmi {
 constexpr int kLdsHistBytes = 131072;    // histogram words in LDS at most
 constexpr int kLdsHistU32Bytes = 65536;  // u32 counts up to this, u16 pairs above
 constexpr int kMaxParticlesPerGroup16 = 65535;
-// slice counts up to which a small bunch takes smaller workgroups
+// slice counts up to which a small bunch takes smaller workgroups: there the
+// counts have four copies; with one, more workgroups meet in its bins (512
+// threads in place of 1024, 2e5 macroparticles: 1024 slices 12.5 us a turn
+// either way, 1100 slices 14.0 -> 15.9)
 constexpr int kSmallBlockSlices = 1024;
 // turns a plain-tracking launch takes at most, by default (odd)
 constexpr int kTurnBlockDefault = 25;
@@ -214,10 +217,11 @@ struct Engine {
     int launch_turns(hipStream_t s, int count, bool advance);
     int finish_chunk(hipStream_t s, int count);
     int launch_turn_kernel(hipStream_t s, int off, bool interp, const KernelEvents &ev);
-    // whether plain turns may run several to a launch (nothing observes the
-    // coordinates or the histogram between turns), and the turns of the
+    // whether nothing observes the coordinates or the histogram between turns,
+    // whether they may then run several to a launch, and the turns of the
     // next launch of a chunk with `left` turns to go (odd, so the last turn's
     // counts use the buffer parity a launch a turn would use)
+    bool plain_turns() const;
     bool multi_turn_ok() const;
     int multi_turn_piece(int left) const;
     int launch_turns_block(hipStream_t s, int off, int turns, const KernelEvents &ev);

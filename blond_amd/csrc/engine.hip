@@ -1245,17 +1245,31 @@ int Engine::get_turn(int *turn) {
 }
 
 // The particle kernels' workgroup: the size the caller gave, or else 1024
-// threads, halved down to 256 while a thread still takes at most two pairs, so
-// that a small bunch
-// spreads over all CUs (moderate slice counts: with few threads the table's
-// staging and the histogram's clearing would dominate).  Turn kernel with 500
-// slices, 1024 threads against this: 5e4 macroparticles 6.4 / 5.1 us, 2e5 7.0 /
-// 6.4 us, 5e5 8.9 / 7.5 us.
+// threads, less for a small bunch, which that spreads over all CUs.  Up to
+// kSmallBlockSlices slices, where every workgroup's own work (the histogram's
+// clearing and flush, the table's staging) is short.  us a turn with 1024, 512
+// and 256 threads:
+//   several turns a launch (or no histogram): halved to 256 while a thread has
+//     at most two pairs; 1000 slices, 1e4 macroparticles 2.13, 1.55, 1.29,
+//     2.5e5 2.23, 1.71, 1.39, 4e5 2.31, 1.74, 1.90, 5.2e5 2.42, 1.73, 1.91
+//   a turn a launch: 512 while a thread has at most one pair; 500 slices,
+//     induced voltage, 6e4 macroparticles 12.3, 11.2, 11.6, 1.5e5 12.5, 12.0,
+//     12.6, 2.5e5 12.6, 12.7, 13.2, 5.2e5 13.9, 14.1, 14.8
+//   the same in FP64 without a table and for 6.5e4 macroparticles at most: 256;
+//     100 slices, 1e4 7.1, 7.0, 6.0, 500 slices, 3e4 7.2, 6.7, 6.5
+//   FP32 with a table: 1024; 1000 slices, 6e4 11.3, 11.3, 12.5, 2.5e5 12.0,
+//     12.5, 13.6
 int Engine::launch_block() const {
+    if (!block_auto || n_slices > kSmallBlockSlices) return block_size;
     const int64_t wgs = (int64_t)device_cu_count() * blocks_per_cu, pairs = (n + 1) / 2;
     int b = block_size;
-    while (block_auto && n_slices <= kSmallBlockSlices && b >= 512 && pairs <= wgs * b) b /= 2;
-    return b;
+    if (n_slices == 0 || plain_turns()) {
+        while (b >= 512 && pairs <= wgs * b) b /= 2;
+        return b;
+    }
+    const bool table = intensity || interp_rf;
+    if ((table && f32) || pairs > wgs * 512) return b;
+    return std::min(b, !table && !f32 && pairs <= wgs * 128 ? 256 : 512);
 }
 
 // The u16-row intensity kernels take buffer descriptors (turn_kernel NEAR)
@@ -1731,10 +1745,13 @@ static int launch_turns_t(const Engine &e, T *x, T *de, const T *rf, const T *ac
     return blmi_check_launch("turns");
 }
 
+bool Engine::plain_turns() const {
+    return turn_block > 1 && !intensity && !interp_rf && !fb_on && !stats_on && !ordered() &&
+           !wake_on() && n_slices > 0 && d_counts;
+}
+
 bool Engine::multi_turn_ok() const {
-    if (turn_block < 2 || intensity || interp_rf || fb_on || stats_on || ordered() || wake_on())
-        return false;
-    if (n_slices <= 0 || !d_counts) return false;
+    if (!plain_turns()) return false;
     int grid = 0;
     size_t lds = 0;
     return hist_layout(launch_block(), &grid, &lds) <= 1;

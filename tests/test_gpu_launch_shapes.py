@@ -56,17 +56,49 @@ def test_intensity_turn_launch_shapes(name, block, per_cu, groups):
 
 
 def test_a_given_block_is_kept():
-    """5000 macroparticles on 100 slices: 256 threads where nothing was given,
-    else what was, the default's value among it."""
-    for given, want in (({}, 256), (dict(block=1024), 1024), (dict(block=512), 512),
-                        (dict(block=64, blocks_per_cu=2), 64)):
-        for name in ("c1", "c2"):
+    """5000 macroparticles on 100 slices: fewer threads where nothing was
+    given, else what was, the default's value among it."""
+    for given, plain, table in (({}, 256, 512), (dict(block=1024), 1024, 1024),
+                                (dict(block=512), 512, 512),
+                                (dict(block=64, blocks_per_cu=2), 64, 64)):
+        for name, want in (("c1", plain), ("c2", table)):
             w = build_workload(name, n_particles=5000, n_turns=4, n_slices=100,
                                **({} if name == "c1" else dict(n_fft=200)))
             assert _shape(w.fused(2, **given)) == (want, given.get("blocks_per_cu", 1))
     # many macroparticles or many slices: the default's full size
     for kw in (dict(n_particles=1_100_000, n_slices=100), dict(n_particles=5000, n_slices=2000)):
         assert _shape(build_workload("c1", n_turns=4, **kw).fused(1)) == (1024, 1)
+
+
+# macroparticles a CU at the edges of each form's rule, and the threads either
+# side: plain turns several and one to a launch, with moments, and a table
+@pytest.mark.parametrize("name,precision,launch,at,low,high", [
+    ("c1", "double", {}, 1024, 256, 512), ("c1", "double", {}, 2048, 512, 1024),
+    ("c1", "single", {}, 1024, 256, 512),
+    ("c1", "double", dict(turn_block=1), 256, 256, 512),
+    ("c1", "double", dict(turn_block=1), 1024, 512, 1024),
+    ("c1", "double", dict(statistics=True), 1024, 512, 1024),
+    ("c1", "single", dict(turn_block=1), 256, 512, 512),
+    ("c2", "double", {}, 1024, 512, 1024), ("c2", "single", {}, 1024, 1024, 1024)])
+def test_block_rule_edges(name, precision, launch, at, low, high):
+    from blond_amd.utils import bm
+
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    bm.use_precision(precision)
+    try:
+        for n, want in ((cus * at, low), (cus * at + 1, high)):
+            out = []
+            for given in ({}, dict(block=1024)):
+                w = build_workload(name, n_particles=n, n_turns=4, n_slices=300,
+                                   **({} if name == "c1" else dict(n_fft=600)))
+                ft = w.fused(3, **launch, **given)
+                assert _shape(ft)[0] == given.get("block", want)
+                out.append((w.beam.dt, w.beam.dE, w.profile.n_macroparticles))
+            # counts are whole numbers and a macroparticle's arithmetic its own
+            for a, b in zip(*out):
+                assert torch.equal(a, b)
+    finally:
+        bm.use_precision("double")
 
 
 def _shape(ft):
