@@ -41,6 +41,53 @@ def test_same_bits_as_the_gathering_kernel(name, n_slices, n_fft, n, precision):
         bm.use_precision("double")
 
 
+# the other drifts, and moments (their sums run over the pairs the byte offsets
+# own, and over the odd last pair and macroparticle), on the line and off it
+@pytest.mark.parametrize("name,n_slices,n_fft", [("c2", 20000, 20000), ("c3", 65536, 131072)])
+@pytest.mark.parametrize("n", [300001, 2 * 262144 + 2, 4 * 262144 + 3])
+@pytest.mark.parametrize("solver,statistics,moved", [
+    ("legacy", False, False), ("exact", False, False), ("simple", True, False),
+    ("exact", True, True)])
+@pytest.mark.parametrize("precision", ["double", "single"])
+def test_same_bits_with_other_drifts_and_moments(name, n_slices, n_fft, n, solver, statistics,
+                                                 moved, precision):
+    bm.use_precision(precision)
+    try:
+        out = []
+        for peel in (0, 1):
+            w = build_workload(name, n_particles=n, n_turns=5, n_slices=n_slices, n_fft=n_fft)
+            w.tracker.solver = solver
+            if moved:
+                w.profile.bin_centers[n_slices // 2:n_slices // 2 + 50] += \
+                    0.1 * float(w.profile.bin_size)
+            ft = w.fused(3, max_peel=peel, statistics=statistics)
+            out.append([a.cpu().numpy() for a in (w.beam.dt, w.beam.dE,
+                                                  w.profile.n_macroparticles,
+                                                  w.tiv.induced_voltage)])
+            if statistics:
+                out[-1].append(ft.statistics(1, 3))
+                assert (out[-1][-1][:, 0] == n).all()
+        for a, b in zip(*out):
+            assert np.array_equal(a, b)
+    finally:
+        bm.use_precision("double")
+
+
+def test_same_bits_beyond_the_last_level_cache():
+    """2^24 macroparticles and three: non-temporal coordinates, on the line
+    and then off it."""
+    ws = [build_workload("c3", n_particles=2 ** 24 + 3, n_turns=5, n_slices=65536, n_fft=131072)
+          for _ in range(2)]
+    for turns, moved in ((2, False), (1, True)):
+        for peel, w in enumerate(ws):
+            if moved:
+                w.profile.bin_centers[32700:32800] += 0.1 * float(w.profile.bin_size)
+            w.fused(turns, max_peel=peel)
+        for get in (lambda w: w.beam.dt, lambda w: w.beam.dE,
+                    lambda w: w.profile.n_macroparticles, lambda w: w.tiv.induced_voltage):
+            assert torch.equal(get(ws[0]), get(ws[1]))
+
+
 # fewer threads stage the window, in more rounds and with the last round cut
 # short; at 20000 slices it starts at an odd bin
 @pytest.mark.parametrize("name,n_slices,n_fft", [("c2", 20000, 20000), ("c3", 65536, 131072)])
