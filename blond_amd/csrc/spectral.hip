@@ -649,8 +649,13 @@ __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
     double *q = conv_lds;                  // q[pad(m)], zero for m >= ns
     double *wv = conv_lds + conv_pad(nq);  // wv[pad(k)] = gl[i0 + k], k < nq + C
     // up to a span of 2048 samples both parities' counts are read and the
-    // turn's chosen when they arrive, so the turn's load is not waited for first
+    // turn's chosen when they arrive, so the turn's load is not waited for
+    // first, and four copies of the counts at a time; beyond, where there is
+    // one copy by default, two: the 512-thread shape then takes 116 registers
+    // and not 170, and two workgroups fit a CU (4096 slices with the beam phase
+    // loop are 264 workgroups: 8.7 -> 6.7 us)
     constexpr bool kBoth = kSpan <= 2048;
+    constexpr int kCopies = kBoth ? 4 : 2;
     const unsigned *cin = nullptr;
     unsigned *cclr = nullptr;
     bool odd = false;
@@ -663,7 +668,7 @@ __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
     // (window, profile, and the window's last C entries with the last batch)
     // is issued before the first LDS store, with clamped in-bounds indexes
     // and the out-of-range values replaced afterwards, so the batch costs
-    // one memory round trip (four copies of the counts at a time).
+    // one memory round trip (and one more for each kCopies copies of the counts).
     constexpr int kStage = 8;
     for (int b = 0; b < nq; b += kStage * TH) {
         double wx[kStage], qx[kStage];
@@ -705,7 +710,8 @@ __global__ void __launch_bounds__(TH) induced_direct_kernel(InducedArgs a) {
 #pragma unroll
             for (int u = 0; u < kStage; ++u) cs[u] = 0u;
             int g = 0;
-            for (; g + 4 <= a.groups; g += 4) copies(std::integral_constant<int, 4>{}, g);
+            for (; g + kCopies <= a.groups; g += kCopies)
+                copies(std::integral_constant<int, kCopies>{}, g);
             for (; g < a.groups; ++g) copies(std::integral_constant<int, 1>{}, g);
 #pragma unroll
             for (int u = 0; u < kStage; ++u) qx[u] = (double)cs[u];

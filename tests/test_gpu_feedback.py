@@ -115,6 +115,18 @@ def test_feedback_turns_fused(kind):
     _check(w, ref)
 
 
+# the loop's workgroups beside 512-thread ones of the convolution, fewer and
+# more than one a CU, with the counts' copies read in twos and singly
+@pytest.mark.parametrize("n_slices", (1100, 3952, 4096))
+@pytest.mark.parametrize("groups", (2, 5))
+def test_loop_beside_the_convolution(n_slices, groups):
+    w = build_feedback_workload("LHC_F", n_particles=40001, n_turns=20, n_slices=n_slices,
+                                intensity=True)
+    ref = _ref(w, 12)
+    w.fused(12, groups=groups)
+    _check(w, ref)
+
+
 @pytest.mark.parametrize("n_slices", (1024, 4096))
 @pytest.mark.parametrize("kind", ("LHC", "LHC_F", "PSB"))
 def test_feedback_turns_fused_with_intensity(kind, n_slices):
