@@ -869,17 +869,28 @@ static int launch_direct_shape(const InducedArgs &a0, hipStream_t s, const Kerne
 //   2000 slices (16, 512, 8) 4.9 us, (16, 256, 8) 5.1
 //   4096 slices (16, 512, 8) 5.5 us, (16, 256, 8) 6.4, (8, 512, 8) 8.2
 //   8192 slices (32, 512, 16)
-//   a multi-turn memory, 16384 outputs of 4096 slices with the wake step:
-//     (32, 256, 16) 10.3 us, (32, 512, 8) 13.3, (16, 512, 8) 19.6: the
-//     exchange of a workgroup's sums is paid for once per 32 outputs and
-//     wavefront, so fewer wavefronts with more samples each
+//   a multi-turn memory (more outputs than slices), with the wake step:
+//     up to 1024 slices (8, 128, 8) while its workgroups, four a CU, all run at
+//     once, above that (32, 128, 8), which does up to four times the outputs:
+//     1000 slices, 5000 outputs 6.5, 6.6 us, 8000 7.0, 6.6, 9000 9.6, 6.6,
+//     20000 14.6, 7.5 ((16, 256, 8): 7.2, 7.5, 9.4, 14.8)
+//     up to 4096 slices (32, 256, 16): 16384 outputs of 4096 slices 10.3 us,
+//     (32, 512, 8) 13.3, (16, 512, 8) 19.6: the exchange of a workgroup's sums
+//     is paid for once per 32 outputs and wavefront, so fewer wavefronts with
+//     more samples each
+//     above, where LDS holds one workgroup a CU, (32, 512, 8): 10000 outputs of
+//     5000 slices 13.6 us, (32, 256, 16) 17.1, (32, 512, 16) 14.9
 int launch_induced_direct(const InducedArgs &a, hipStream_t s, const KernelEvents &ev) {
     if (!a.gl || a.n_slices < 1 || a.n_out < a.n_slices ||
         (int64_t)a.n_out + a.n_slices - 1 > a.gl_len ||
         (a.tab && a.n_out != a.n_slices && !a.with_wake) ||
         (a.with_wake && (a.wk.n_mem > a.n_out || (a.wk.ind_coef && a.n_slices < 2))))
         return blmi_set_error(BLMI_ERR_ARG, "direct induced voltage: bad arguments");
-    if (a.n_out > a.n_slices && a.n_slices > 1024) return launch_direct_shape<32, 256, 16>(a, s, ev);
+    if (a.n_out > a.n_slices) {
+        if (a.n_slices > 4096) return launch_direct_shape<32, 512, 8>(a, s, ev);
+        if (a.n_slices > 1024) return launch_direct_shape<32, 256, 16>(a, s, ev);
+        if (a.n_out > 8 * 4 * device_cu_count()) return launch_direct_shape<32, 128, 8>(a, s, ev);
+    }
     if (a.n_slices <= 1024)
         return a.with_fb ? launch_direct_shape<16, 256, 8>(a, s, ev)
                          : launch_direct_shape<8, 128, 8>(a, s, ev);

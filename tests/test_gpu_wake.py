@@ -117,6 +117,31 @@ def test_wake_first_turn_fused_exact_profile(kind):
     _check_sources(w, ref)
 
 
+# memories at the edges of the direct convolution's shapes: 8 outputs a
+# workgroup up to 8192 of them and 32 above (256 CUs), 1024 and 4096 slices,
+# the largest memory of 2^26 products and a fraction of a workgroup's outputs;
+# a memory of more than 20480 points is formed by the four-step transform
+@pytest.mark.parametrize("n_slices,memory", [(1024, 8), (911, 9), (1024, 9), (64, 129),
+                                             (1000, 20), (1000, 33), (1025, 2), (4096, 2),
+                                             (4097, 2), (5792, 2)])
+@pytest.mark.parametrize("kind", ["mtw", "mtw_front"])
+def test_memory_shapes(n_slices, memory, kind):
+    """Two turns: the second shifts the first's memory.  The first's profile is
+    exact, the voltage and the memory to 1e-10 of their maximum after each."""
+    w = build_wake_workload(kind, n_particles=40001, n_turns=4, n_slices=n_slices,
+                            memory_turns=memory)
+    for turns in (1, 1):
+        ref = orc.track(w.snapshot(), turns)
+        ft = w.fused(turns)
+        assert ft.method == ("direct" if n_slices * memory <= 20480 else "fourstep")
+        np.testing.assert_array_equal(host(w.profile.n_macroparticles), ref["profile"])
+        v = host(w.tiv.induced_voltage)
+        assert np.abs(v - ref["induced_voltage"]).max() <= 1e-10 * np.abs(ref["induced_voltage"]).max()
+        sc = np.abs(ref["dE"]).max()
+        np.testing.assert_allclose(host(w.beam.dE), ref["dE"], rtol=0, atol=1e-12 * sc)
+        _check_sources(w, ref)
+
+
 CONV_KINDS = ("mtw", "mtw_front", "mtw_time", "mixed")
 
 
