@@ -975,6 +975,8 @@ int Adjoint::init(int64_t n_, int n_rf_, int n_turns_, int n_slices_, int every_
 int Adjoint::set_particles(const double *dt, const double *dE) {
     BLMI_HIP_TRY(hipMemcpy(d_x0, dt, sizeof(double) * n, hipMemcpyDeviceToDevice));
     BLMI_HIP_TRY(hipMemcpy(d_x0 + np, dE, sizeof(double) * n, hipMemcpyDeviceToDevice));
+    // a pass enqueued from a stream that does not wait for the default one
+    BLMI_HIP_TRY(hipStreamSynchronize(nullptr));
     forward_done = false;
     return BLMI_OK;
 }
@@ -985,6 +987,8 @@ int Adjoint::set_programs(const double *rf_host, const double *acc_host, const d
                           const double *alpha1, const double *alpha2, const double *beta,
                           const double *energy, double charge_) {
     const size_t nt = (size_t)n_turns + 1;
+    // a pass in flight (a forward without its backward) reads the programs
+    if (own) BLMI_HIP_TRY(hipStreamSynchronize(own));
     // the captured passes hold scalars by value: a changed one re-captures
     if (charge_ != charge) invalidate_graphs();
     charge = charge_;
@@ -1035,6 +1039,7 @@ int Adjoint::set_wake(int64_t n_fft_, const double *g_host, double scale_) {
     if (n_fft_ < n_slices || n_fft_ > 8192)
         return blmi_set_error(BLMI_ERR_UNSUPPORTED, "adjoint: n_fft %lld outside [n_slices, 8192]",
                               (long long)n_fft_);
+    if (own) BLMI_HIP_TRY(hipStreamSynchronize(own));  // as set_programs
     if (n_fft_ != n_fft || scale_ != scale) invalidate_graphs();
     if (n_fft_ != n_fft) {
         (void)hipFree(d_g);

@@ -1228,6 +1228,9 @@ void Engine::invalidate_graph() {
 int Engine::set_turn(int turn) {
     if (turn < 0 || turn >= n_turns)
         return blmi_set_error(BLMI_ERR_ARG, "turn %d outside [0, %d)", turn, n_turns);
+    // turns in flight on the engine's stream read what is set here, and turns
+    // enqueued from a stream that does not wait for the default one use it
+    BLMI_HIP_TRY(hipStreamSynchronize(own_stream));
     BLMI_HIP_TRY(hipMemcpy(d_base, &turn, sizeof(int), hipMemcpyHostToDevice));
     host_turn = turn;
     // staged counts refer to the old turn: drop them (prime rebuilds them)
@@ -1236,6 +1239,7 @@ int Engine::set_turn(int turn) {
                                sizeof(unsigned) * 2 * (size_t)groups * (size_t)n_slices));
     BLMI_HIP_TRY(hipMemset(d_base + 1, 0xff, sizeof(int) * 2));
     BLMI_HIP_TRY(hipMemset(line_flags(), 0, sizeof(int) * 2));
+    BLMI_HIP_TRY(hipStreamSynchronize(nullptr));
     return BLMI_OK;
 }
 
