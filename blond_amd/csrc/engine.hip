@@ -1231,15 +1231,14 @@ int Engine::set_turn(int turn) {
     // turns in flight on the engine's stream read what is set here, and turns
     // enqueued from a stream that does not wait for the default one use it
     BLMI_HIP_TRY(hipStreamSynchronize(own_stream));
-    BLMI_HIP_TRY(hipMemcpy(d_base, &turn, sizeof(int), hipMemcpyHostToDevice));
-    host_turn = turn;
     // staged counts refer to the old turn: drop them (prime rebuilds them)
     if (d_counts)
         BLMI_HIP_TRY(hipMemset(d_counts, 0,
                                sizeof(unsigned) * 2 * (size_t)groups * (size_t)n_slices));
-    BLMI_HIP_TRY(hipMemset(d_base + 1, 0xff, sizeof(int) * 2));
-    BLMI_HIP_TRY(hipMemset(line_flags(), 0, sizeof(int) * 2));
+    const int words[5] = {turn, -1, -1, 0, 0};
+    BLMI_HIP_TRY(hipMemcpy(d_base, words, sizeof(words), hipMemcpyHostToDevice));
     BLMI_HIP_TRY(hipStreamSynchronize(nullptr));
+    host_turn = turn;
     return BLMI_OK;
 }
 

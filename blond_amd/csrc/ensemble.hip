@@ -420,11 +420,11 @@ int Ensemble::set_turn(int turn) {
         return blmi_set_error(BLMI_ERR_ARG, "turn %d outside [0, %d)", turn, n_turns);
     // as Engine::set_turn
     BLMI_HIP_TRY(hipStreamSynchronize(own_stream));
-    BLMI_HIP_TRY(hipMemcpy(d_base, &turn, sizeof(int), hipMemcpyHostToDevice));
-    host_turn = turn;
     if (d_counts)
         BLMI_HIP_TRY(hipMemset(d_counts, 0, sizeof(unsigned) * (size_t)n_bunches * n_slices));
+    BLMI_HIP_TRY(hipMemcpy(d_base, &turn, sizeof(int), hipMemcpyHostToDevice));
     BLMI_HIP_TRY(hipStreamSynchronize(nullptr));
+    host_turn = turn;
     return BLMI_OK;
 }
 
