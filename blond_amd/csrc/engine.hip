@@ -1795,7 +1795,6 @@ InducedArgs Engine::induced_args(int off) const {
     ia.tab = reinterpret_cast<double2 *>(d_table);
     ia.tab_params = d_table + 2 * n_slices;
     ia.f32 = f32 ? 1 : 0;
-    ia.line = bin_line_args();
     int ps = 31, pl = 0, m1lo = 0;
     ia.part = nullptr;
     ia.cnt_out = nullptr;
@@ -1850,14 +1849,14 @@ int Engine::launch_induced(hipStream_t s, int off, const KernelEvents &ev) {
             ia.fb.from_counts = 1;  // the profile is being written beside it
         }
         int rc = method == 1   ? launch_induced_direct(ia, s, e1)
-                 : method == 2 ? launch_induced_fourstep(ia, plan2, s, e1)
+                 : method == 2 ? launch_induced_fourstep(ia, plan2, s, e1, bin_line_args())
                                : launch_induced_voltage_lds(ia, plan, s, e1);
         if (rc || !w) return rc;
     }
     KernelEvents e2;
     e2.start = have_conv ? nullptr : ev.start;
     e2.stop = ev.stop;
-    return launch_wake_finish(wake_args(off), s, e2);
+    return launch_wake_finish(wake_args(off), s, e2, bin_line_args());
 }
 
 int Engine::set_feedback(int machine, int delay, int first_bin, double alpha, double reference,
@@ -2026,7 +2025,6 @@ WakeArgs Engine::wake_args(int off) const {
     a.volt = volt;
     a.tab = reinterpret_cast<double2 *>(d_table);
     a.tab_params = d_table + 2 * n_slices;
-    a.line = bin_line_args();
     return a;
 }
 

@@ -64,7 +64,6 @@ struct InducedArgs {
     double2 *tab;
     double *tab_params;
     int f32;          // table in the reference's single-precision arithmetic
-    BinLine line;     // four-step method: the table's bin centres against the cuts' line
     // four-step method: the profile as the sum of part_rows u16-pair rows
     // stored transposed (column m2's word m1 of row r at
     // part[(m2 part_rows + r) 2^part_lshift + m1]); nullptr: the counts
@@ -139,8 +138,12 @@ void fft2_plan_destroy(Fft2Plan *plan);
 void fft2_permute_z(const Fft2Plan &p, const double2 *Z_host, double2 *Zp_host);
 // Same contract as launch_induced_voltage_lds (InducedArgs, including the
 // interpolation table).  `ev`, when given, spans the three
-// launches (start at pass A, stop at pass C).
+// launches (start at pass A, stop at pass C).  Pass C compares the table's bin
+// centres with `line` where that has flags (an argument of its own: in
+// InducedArgs, which the direct convolution's launches carry too, it cost those
+// with the beam phase loop 0.2 us).
 int launch_induced_fourstep(const InducedArgs &a, const Fft2Plan &p, hipStream_t s,
-                            const KernelEvents &ev = KernelEvents());
+                            const KernelEvents &ev = KernelEvents(),
+                            const BinLine &line = BinLine{});
 
 }  // namespace blmi

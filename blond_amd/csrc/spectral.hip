@@ -1402,7 +1402,8 @@ template <int FL>
 __global__ void __launch_bounds__(kColThreads) fft2_c_kernel(InducedArgs a, int M1, int M2,
                                                              int cols, StageList st1,
                                                              const double2 *__restrict__ twM,
-                                                             const double2 *__restrict__ S) {
+                                                             const double2 *__restrict__ S,
+                                                             BinLine line) {
     extern __shared__ double2 buf[];
     const int NC = cols + 1;
     const int ld = M1 + 1;
@@ -1452,7 +1453,7 @@ __global__ void __launch_bounds__(kColThreads) fft2_c_kernel(InducedArgs a, int 
         if (2 * m + 1 < a.n_out) a.volt[2 * m + 1] = v1;
         if (a.tab && 2 * m < ns - 1) {
             const double b0 = one ? bc_pre[0] : a.bc[2 * m];
-            off |= a.line.off(2 * m, b0);
+            off |= line.off(2 * m, b0);
             store_interp_entry(a.tab, 2 * m, interp_entry(v0, v1, b0, a.charge, inv_bw, a.f32),
                                a.f32);
             if (2 * m + 1 < ns - 1) {
@@ -1461,14 +1462,14 @@ __global__ void __launch_bounds__(kColThreads) fft2_c_kernel(InducedArgs a, int 
                                    : buf[cols * ld + (last ? m1 + 1 : m1)];
                 const double v2 = -(a.scale * (un.x * fct));
                 const double b1 = one ? bc_pre[1] : a.bc[2 * m + 1];
-                off |= a.line.off(2 * m + 1, b1);
+                off |= line.off(2 * m + 1, b1);
                 store_interp_entry(a.tab, 2 * m + 1,
                                    interp_entry(v1, v2, b1, a.charge, inv_bw, a.f32), a.f32);
             }
         }
     }
-    if (a.line.flags)
-        a.line.put(off, *a.turn_base + a.turn_off, blockIdx.x == 0 && threadIdx.x == 0);
+    if (line.flags)
+        line.put(off, *a.turn_base + a.turn_off, blockIdx.x == 0 && threadIdx.x == 0);
 }
 
 static bool factor_list(int L, int *radix, int &n) {
@@ -1632,7 +1633,7 @@ static Fft2Kernels fft2_kernels(int M1, int M2) {
 }
 
 int launch_induced_fourstep(const InducedArgs &a, const Fft2Plan &p, hipStream_t s,
-                            const KernelEvents &ev) {
+                            const KernelEvents &ev, const BinLine &line) {
     if (!p.M) return blmi_set_error(BLMI_ERR_ARG, "four-step plan not created");
     if (a.n_slices > p.n_real || a.n_out < 0 || a.n_out > p.n_real)
         return blmi_set_error(BLMI_ERR_ARG, "n_slices %d / n_out %d exceed n_fft %d", a.n_slices,
@@ -1665,7 +1666,7 @@ int launch_induced_fourstep(const InducedArgs &a, const Fft2Plan &p, hipStream_t
     hipLaunchKernelGGL(k.b, dim3(p.M1 / 2 + 1), dim3(p.threads_b), lds_b, s, a, p.M1,
                        p.M2, st2, p.twM, p.twB, p.T, p.S);
     launch(k.c, dim3(cols), dim3(kColThreads), lds_c, s, last, a, p.M1, p.M2, p.cols,
-           st1, p.twM, p.S);
+           st1, p.twM, p.S, line);
     return blmi_check_launch("induced_fourstep");
 }
 

@@ -165,9 +165,10 @@ struct WakeArgs {
     double *volt;
     double2 *tab;           // (slope, intercept) per bin, tab_params = (bc[0], inv_bw)
     double *tab_params;
-    BinLine line;           // wake_finish: the table's bin centres against the cuts' line
 };
-int launch_wake_finish(const WakeArgs &a, hipStream_t s, const KernelEvents &ev = KernelEvents());
+// The table's bin centres are compared with `line` where that has flags.
+int launch_wake_finish(const WakeArgs &a, hipStream_t s, const KernelEvents &ev = KernelEvents(),
+                       const BinLine &line = BinLine{});
 // memory[(*turn_base) & 1] -> out[n_mem] (publish the current memory)
 int launch_mtw_publish(const int *turn_base, const double *mem0, const double *mem1, int64_t n_mem,
                        double *out, hipStream_t s);

@@ -89,7 +89,7 @@ int launch_mtw_shift_add(const double *mem_in, double *mem_out, const double *ti
 // ---------------------------------------------------------------------------
 // engine finishing step
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kWakeBlock) wake_finish_kernel(WakeArgs a) {
+__global__ void __launch_bounds__(kWakeBlock) wake_finish_kernel(WakeArgs a, BinLine line) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int t = *a.turn_base + a.turn_off;
     const int ns = a.n_slices;
@@ -145,17 +145,18 @@ __global__ void __launch_bounds__(kWakeBlock) wake_finish_kernel(WakeArgs a) {
             const double vn = total_at((int)i + 1);
             const double k = a.charge * (vn - vi) * inv_bw;
             a.tab[i] = make_double2(k, (a.charge * vi - a.bc[i] * k) + 0.0);
-            off = a.line.off((int)i, a.bc[i]);
+            off = line.off((int)i, a.bc[i]);
         }
     }
-    a.line.put(off, t, i == 0);
+    line.put(off, t, i == 0);
 }
 
-int launch_wake_finish(const WakeArgs &a, hipStream_t s, const KernelEvents &ev) {
+int launch_wake_finish(const WakeArgs &a, hipStream_t s, const KernelEvents &ev,
+                       const BinLine &line) {
     const int64_t n = a.n_mem > a.n_slices ? a.n_mem : (int64_t)a.n_slices;
     if (a.ind_coef && a.n_slices < 2)
         return blmi_set_error(BLMI_ERR_ARG, "inductive source: at least 2 slices");
-    launch(wake_finish_kernel, dim3(grid_for(n)), dim3(kWakeBlock), 0, s, ev, a);
+    launch(wake_finish_kernel, dim3(grid_for(n)), dim3(kWakeBlock), 0, s, ev, a, line);
     return blmi_check_launch("wake_finish");
 }
 
