@@ -56,6 +56,8 @@ struct Adjoint {
     // the forward and reverse passes are captured once per turn count and
     // replayed as HIP graphs on the adjoint's own stream
     hipStream_t own = nullptr;
+    bool in_flight = false;  // a forward pass nobody has waited for yet
+    int settle();            // wait for it
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
     hipGraphExec_t fwd_exec = nullptr, bwd_exec = nullptr;
     int fwd_graph_turns = -1, bwd_graph_turns = -1;

@@ -919,6 +919,12 @@ int Adjoint::ensure_stream() {
     return BLMI_OK;
 }
 
+int Adjoint::settle() {
+    if (in_flight) BLMI_HIP_TRY(hipStreamSynchronize(own));
+    in_flight = false;
+    return BLMI_OK;
+}
+
 void Adjoint::release() {
     invalidate_graphs();
     if (own) (void)hipStreamDestroy(own);
@@ -987,8 +993,8 @@ int Adjoint::set_programs(const double *rf_host, const double *acc_host, const d
                           const double *alpha1, const double *alpha2, const double *beta,
                           const double *energy, double charge_) {
     const size_t nt = (size_t)n_turns + 1;
-    // a pass in flight (a forward without its backward) reads the programs
-    if (own) BLMI_HIP_TRY(hipStreamSynchronize(own));
+    int rc = settle();  // a forward without its backward reads the programs
+    if (rc) return rc;
     // the captured passes hold scalars by value: a changed one re-captures
     if (charge_ != charge) invalidate_graphs();
     charge = charge_;
@@ -1039,7 +1045,8 @@ int Adjoint::set_wake(int64_t n_fft_, const double *g_host, double scale_) {
     if (n_fft_ < n_slices || n_fft_ > 8192)
         return blmi_set_error(BLMI_ERR_UNSUPPORTED, "adjoint: n_fft %lld outside [n_slices, 8192]",
                               (long long)n_fft_);
-    if (own) BLMI_HIP_TRY(hipStreamSynchronize(own));  // as set_programs
+    int rc = settle();  // as set_programs
+    if (rc) return rc;
     if (n_fft_ != n_fft || scale_ != scale) invalidate_graphs();
     if (n_fft_ != n_fft) {
         (void)hipFree(d_g);
@@ -1227,6 +1234,7 @@ int Adjoint::forward(int turns, double *profile_out, hipStream_t user) {
     }
     BLMI_HIP_TRY(hipEventRecord(ev_in, user));
     BLMI_HIP_TRY(hipStreamWaitEvent(own, ev_in, 0));
+    in_flight = true;
     BLMI_HIP_TRY(hipGraphLaunch(fwd_exec, own));
     BLMI_HIP_TRY(hipMemcpyAsync(profile_out, d_prof + (size_t)turns * n_slices,
                                 sizeof(double) * n_slices, hipMemcpyDeviceToDevice, own));
@@ -1261,6 +1269,7 @@ int Adjoint::backward(const double *dprofile, double *grad_rf_host, double *corr
     BLMI_HIP_TRY(hipMemcpyAsync(corr_host, d_corr, sizeof(double) * n_fft, hipMemcpyDeviceToHost,
                                 own));
     BLMI_HIP_TRY(hipStreamSynchronize(own));
+    in_flight = false;
     for (int j = 0; j < 2 * n_rf; ++j) {
         double v = 0.0;
         for (int b = 0; b < grid; ++b) v += gp[(size_t)b * 2 * n_rf + j];
