@@ -1078,6 +1078,10 @@ struct LdsKernels {
     bool stage = false;  // twiddles in LDS
 };
 
+// Twiddles in LDS wherever they fit beside the data: a batch's launch with 16,
+// 256 and 600 bunches of 300 slices 11.0, 13.2, 23.9 -> 9.9, 10.9, 21.1 us, of
+// 1000 slices 12.3, 15.9, 29.3 -> 10.9, 13.2, 25.4, of 2000 slices 16.5, 21.0,
+// 40.2 -> 14.0, 17.5, 35.1 (the second workgroup of a CU still fits).
 static LdsKernels lds_kernels(int M, int threads) {
     LdsKernels k;
     const bool wave = wave_len(M) && threads == kLdsWaveThreads;
