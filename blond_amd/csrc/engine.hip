@@ -268,7 +268,7 @@ constexpr int kBufferFlags = 0x00027000;
 // formed from two voltages with 12 operations more.  A macroparticle outside
 // the window gathers a 128-byte line for its 16 bytes from L2, beside the
 // stream of the coordinates.  Two RF systems, 65536 slices, kernel: 1e7
-// macroparticles 67.6 -> 66.5 us, 3e7 295 -> 241 us (the stream alone at the
+// macroparticles 66.9 -> 62.1 us, 3e7 304 -> 245 us (the stream alone at the
 // rate of an in-place copy: 41 and 175 us); FP32, addresses only, 1e7 45.9 ->
 // 44.5 us.  Measured the same: two pairs more in flight, gathers issued before
 // the stores, part of a 3e7 bunch kept in the last-level cache.
